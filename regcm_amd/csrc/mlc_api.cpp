@@ -595,6 +595,7 @@ int create_handle(const mlc_grid_desc *g, hipStream_t shared, mlc_handle **out) 
     h->s_tr0 = h->nslots;
     for (int n = 0; n < g->ntr; ++n) h->adv_list[h->nadvf++] = h->nslots++;
   }
+  h->tune.wafv_group = wafv_rule(column_waves(h->d), h->nadvf);
   h->h_mx.assign((size_t)h->d.plane, 0.0);
   h->h_mu.assign((size_t)h->d.plane, 0.0);
   h->h_mv.assign((size_t)h->d.plane, 0.0);

@@ -261,6 +261,14 @@ int mlc_batch_create(const mlc_grid_desc *descs, int n, mlc_batch **out) {
     b->groups[0].m.push_back(h);
     b->npoints += mlc_npoints(h);
   }
+  // the members' launches are merged: one choice, by their common grid
+  long long waves = 0;
+  int nf = 0;
+  for (const mlc_handle *h : b->all) {
+    waves += column_waves(h->d);
+    nf = h->nadvf > nf ? h->nadvf : nf;
+  }
+  for (mlc_handle *h : b->all) h->tune.wafv_group = wafv_rule(waves, nf);
   *out = b;
   return MLC_OK;
 }

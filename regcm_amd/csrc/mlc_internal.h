@@ -172,6 +172,33 @@ struct ZMet {
   }
 };
 
+// Fields per thread of the vertical WAF for nf fields on cross columns that
+// make `waves` wavefronts.  A SIMD runs its waves' levels one after the
+// other, and a level costs about 0.7 of a field on top of the fields (s and
+// the metric ratios), so the cost is the waves of the fullest of the chip's
+// 1024 SIMDs times (fields per wave + 0.7): few fields per wave where the
+// domain leaves SIMDs idle or unevenly filled, four where it fills them.
+// Measured, us per call at 4 / 2 / 1: 64x64x23 20.2 / 16.2 / 13.8,
+// 151x127x35 57 / 47 / 53, 500x100x60 144 / 128 / 162, 256x256x41 109 / 128 / 145.
+inline int wafv_rule(long long waves, int nf) {
+  int best = 4;
+  double cost = 0.0;
+  for (int g = 4; g >= 1; g /= 2) {
+    const int groups = (nf + g - 1) / g;
+    const double c = (double)((waves * groups + 1023) / 1024) * ((double)nf / groups + 0.7);
+    if (g == 4 || c < cost) {
+      best = g;
+      cost = c;
+    }
+  }
+  return best;
+}
+
+// Wavefronts of 64 x 1 columns that cover a domain's cross points.
+inline long long column_waves(const Dims &d) {
+  return (long long)((d.je2 + 63) / 64) * ((d.ie2 + 3) / 4) * 4;
+}
+
 // Kernel slots for per-kernel timing.
 enum KernelSlot {
   K_DIV = 0, K_COL, K_MOM, K_STAG_IN, K_WAF_V, K_WAF_H, K_CURV, K_STAG_OUT,
@@ -289,7 +316,7 @@ struct mlc_handle {
     int mom_chunk = 0;           // momentum, if not 0: levels per thread
     int stag_chunk = 1;          // staggering passes: levels per thread
     int column = 2;              // column solve: 0 LDS three-phase, 1 streamed, 2 chunked
-    int wafv_group = 4;          // vertical WAF: fields per thread (1, 2 or 4)
+    int wafv_group = 4;          // vertical WAF: fields per thread (1, 2 or 4; wafv_rule)
     int xcd_map = 1;             // XCD-contiguous tile order of single-domain launches
     int waf_tile = 4;            // LDS-tile WAF: output rows per tile (4 or 8; FP64 starts at 8)
     int waf_hgroup = 0;          // LDS-tile WAF: fields per block (0 = the whole batch)

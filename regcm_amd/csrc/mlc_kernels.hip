@@ -74,9 +74,60 @@ __device__ __forceinline__ R flow_param(R num, R den) {
 }
 
 // b = max(0, min(2, max(r, min(2r, 1))))  (Main/mod_moloch.F90:882)
+// A NaN r gives 1 in either form, and a zero's sign does not reach zphi.
+__device__ __forceinline__ double waf_b(double r) {
+  return fmax(0.0, fmin(2.0, fmax(r, fmin(2.0 * r, 1.0))));
+}
+__device__ __forceinline__ float waf_b(float r) {
+  return fmaxf(0.0f, fminf(2.0f, fmaxf(r, fminf(2.0f * r, 1.0f))));
+}
+
+// num / den as the limiter needs it, for |den| >= FlowLim::den(): correctly
+// rounded between -4 and 4, past them some value of the same sign beyond 2
+// (waf_b takes 2 or 0 there).  The reciprocal is refined by one third-order
+// step (the hardware's is good to 2^-24), the quotient by its exact remainder
+// (Markstein's correction), the special operands by v_div_fixup.  The
+// compiler's own sequence scales both operands against overflow and
+// underflow; here the quotient is held within +-4 before the remainder is
+// formed, and a remainder can lose bits only for |num| below 1e-280 (1e-31 in
+// float), whose quotient is too small to change zphi = 1 + zamu b - b in its
+// last bit.
+__device__ __forceinline__ double waf_ratio(double num, double den) {
+  double y = __builtin_amdgcn_rcp(den);
+  double e = __builtin_fma(-den, y, 1.0);
+  e = __builtin_fma(e, e, e);
+  y = __builtin_fma(y, e, y);
+  const double q = fmax(fmin(num * y, 4.0), -4.0);
+  const double r = __builtin_fma(-den, q, num);
+  return __builtin_amdgcn_div_fixup(__builtin_fma(r, y, q), den, num);
+}
+__device__ __forceinline__ float waf_ratio(float num, float den) {
+  float y = __builtin_amdgcn_rcpf(den);
+  y = __builtin_fmaf(__builtin_fmaf(-den, y, 1.0f), y, y);
+  float q = fmaxf(fminf(num * y, 4.0f), -4.0f);
+  q = __builtin_fmaf(__builtin_fmaf(-den, q, num), y, q);
+  const float r = __builtin_fmaf(-den, q, num);
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(r, y, q), den, num);
+}
+
+// flow_param without a branch: the quotient is formed in every lane and
+// replaced where the denominator is degenerate.
 template <typename R>
-__device__ __forceinline__ R waf_b(R r) {
-  return rmax(R(0), rmin(R(2), rmax(r, rmin(R(2) * r, R(1)))));
+__device__ __forceinline__ R flow_param_sel(R num, R den) {
+  const R q = waf_ratio(num, den);
+  const R z = fabs(num) < FlowLim<R>::num() ? R(1) : R(0);
+  return fabs(den) < FlowLim<R>::den() ? z : q;
+}
+
+// zphi = is + zamu*b - is*b with is = 1 (up) or -1: the same as is times
+// (1 + |zamu|*b - b), sign for sign, since rounding is symmetric.
+__device__ __forceinline__ double waf_phi(double az, double b, bool up) {
+  const double t = (1.0 + az * b) - b;
+  return __hiloint2double(__double2hiint(t) ^ (up ? 0 : (int)0x80000000), __double2loint(t));
+}
+__device__ __forceinline__ float waf_phi(float az, float b, bool up) {
+  const float t = (1.0f + az * b) - b;
+  return __int_as_float(__float_as_int(t) ^ (up ? 0 : (int)0x80000000));
 }
 
 // ---------------------------------------------------------------------------
@@ -960,33 +1011,41 @@ __device__ __forceinline__ void StaggerIn<R>::run(const StaggerIn &args_, int bx
 }
 
 // ---------------------------------------------------------------------------
-// WAF vertical advection, both half steps (:862-922), one column and one
-// field per lane, streamed top to bottom through register windows: the
-// first half step emits wz1(k) once pp(k+2) is loaded, the second emits
+// WAF vertical advection, both half steps (:862-922), one column and up to G
+// fields per lane, streamed top to bottom through register windows: the
+// first half step emits wz1(k) once x(k+2) is loaded, the second emits
 // wz2(k-2) once wz1(k) is known, so every face flux is evaluated once and
 // each input is read once.  zrfmu(k) = dtrdz*fmz(k)/fmzf(k) and
 // zrfmd(k) = dtrdz*fmz(k)/fmzf(k+1) are precomputed at init with exactly
 // these operations.  T is the field/arithmetic type, S the type of s and
 // of the metric ratios.
+//
+// What bounds it: instruction issue, until the domain no longer fits the
+// last-level cache and the 2F + 3 arrays do.  So a face is branch-free, its
+// limiter is min/max instructions, its division leaves out the scaling
+// (waf_ratio) and the parts that do not depend on the field are formed once per
+// level: 47 vector instructions per face instead of 74.  Measured per call,
+// one domain alone: 64x64x23 38.0 -> 13.8 us, 151x127x35 68.1 -> 47.5,
+// 500x100x60 156 -> 128, 256x256x41 FP64 114 -> 109 (4.5 TB/s over its 23
+// arrays) and mixed 83.9 -> 66.3.
 template <typename T>
-__device__ __forceinline__ T waf_vflux(T skp1, T dtrdz, T xm1, T x0, T x1,
-                                       T x2) {
-  // face kk+1 with xm1 = x(max(kk-1,1)), x0 = x(kk), x1 = x(kk+1),
-  // x2 = x(min(kk+2,kz)): the k1/k1p1 clamps of :870-880
-  const T zamu = skp1 * dtrdz;
-  T is, num;
-  if (zamu >= T(0)) {
-    is = T(1);
-    num = x1 - x2;
-  } else {
-    is = T(-1);
-    num = xm1 - x0;
+struct WafFace {       // the field-independent part of a face flux
+  T az, half;          // |s dtrdz|, 0.5 s
+  bool up;             // s dtrdz >= 0
+  __device__ __forceinline__ WafFace(T s, T dtrdz) {
+    const T zamu = s * dtrdz;
+    az = fabs(zamu);
+    half = T(0.5) * s;
+    up = zamu >= T(0);
   }
-  const T r = flow_param(num, x0 - x1);
-  const T b = waf_b(r);
-  const T zphi = is + zamu * b - is * b;
-  return T(0.5) * skp1 * ((T(1) + zphi) * x1 + (T(1) - zphi) * x0);
-}
+  // face kk+1 from xm, x0, x1, x2 = x(kk-1), x(kk), x(kk+1), x(kk+2), with
+  // the k1/k1p1 clamps of :870-880 in the caller's operands
+  __device__ __forceinline__ T flux(T xm, T x0, T x1, T x2) const {
+    const T b = waf_b(flow_param_sel(up ? x1 - x2 : xm - x0, x0 - x1));
+    const T zphi = waf_phi(az, b, up);
+    return half * ((T(1) + zphi) * x1 + (T(1) - zphi) * x0);
+  }
+};
 
 template <typename T, typename S, int G>
 struct WafVertical {
@@ -996,133 +1055,148 @@ struct WafVertical {
   const S * zrfmu;
   const S * zrfmd;
   double dtrdz_;
-  int nf;                      // fields in the batch; a thread takes G of them
+  int nf;                      // fields in the batch
+  int ngroups;                 // bz = 0 .. ngroups-1: near-equal groups of at most G fields
   static __device__ __forceinline__ void run(const WafVertical &args_, int bx, int by, int bz);
 };
 
-// A thread streams the column of G fields (f0 .. f0+G-1, f0 = G*bz) so that
-// the per-level loads of s, zrfmu and zrfmd are shared by the group.
+// The column of the N fields f0 .. f0+N-1; the per-level loads of s, zrfmu
+// and zrfmd are shared by them.  N is a compile-time count, so that a level
+// has no per-field branch.
+template <int N, typename T, typename S>
+__device__ __forceinline__ void waf_column(const Dims &d, const AdvPtrs<T> &ap, const S *s,
+                                           const S *zrfmu, const S *zrfmd, T dtrdz, int f0,
+                                           int j, int i) {
+  const int kz = d.kz;
+  const long long P = d.plane;
+  // a lane's byte offsets in a level (32 bits: a level is far below 4 GiB);
+  // the level's base address is uniform
+  const unsigned ot = (unsigned)d.at2(j, i) * (unsigned)sizeof(T);
+  const unsigned os = (unsigned)d.at2(j, i) * (unsigned)sizeof(S);
+  auto ld = [&](const T *p) { return *(const T *)((const char *)p + ot); };
+  auto lds = [&](const S *p) { return *(const S *)((const char *)p + os); };
+  const T *px[N];              // level k + 3
+  T *po[N];                    // level k - 2
+  // per field: x(k), x(k+1), x(k+2); the differences x(k-1)-x(k) and
+  // x(k)-x(k+1); the flux on the top face of level k; the same of the second
+  // half step, two levels behind, on wz1
+  T xm[N], x0[N], x1[N], x2[N], f1[N], ym[N], y0[N], y1[N], f2[N];
+#pragma unroll
+  for (int g = 0; g < N; ++g) {
+    px[g] = ap.src[f0 + g];
+    po[g] = ap.dst[f0 + g] - 2 * P;
+    x0[g] = ld(px[g]);
+    x1[g] = ld(px[g] + P);
+    x2[g] = ld(px[g] + 2 * P);
+    px[g] += 3 * P;
+  }
+  T s_k = T(lds(s)), s_n = T(lds(s + P));    // s(k), s(k+1)
+  T s_1 = T(0), s_2 = T(0);                  // s(k-1), s(k-2)
+  T u_k = T(lds(zrfmu)), d_k = T(lds(zrfmd)), u_1 = T(0), u_2 = T(0), d_1 = T(0), d_2 = T(0);
+  s += 2 * P;                                // level k + 2
+  zrfmu += P;                                // level k + 1
+  zrfmd += P;
+#pragma unroll
+  for (int g = 0; g < N; ++g) {
+    xm[g] = x0[g];
+    f1[g] = f2[g] = ym[g] = y0[g] = y1[g] = T(0);
+  }
+  // Level k: wz1(k) and, from k = 3 on (emit), wz2(k-2).  The next level's
+  // x, s and metric ratios are requested first, before this level's stores
+  // (a load issued after a store would wait for the store as well).
+  auto level = [&](int k, auto emit_, auto last_) __attribute__((always_inline)) {
+    constexpr bool emit = decltype(emit_)::value, last = decltype(last_)::value;
+    T x3[N];
+    S ns = S(0), nu = S(0), nd = S(0);
+    if constexpr (!last) {
+      // x(min(k+3, kz))
+#pragma unroll
+      for (int g = 0; g < N; ++g) {
+        x3[g] = ld(px[g]);
+        if (k + 3 < kz) px[g] += P;
+      }
+      ns = lds(s);
+      nu = lds(zrfmu);
+      nd = lds(zrfmd);
+      s += P;
+      zrfmu += P;
+      zrfmd += P;
+    }
+    const WafFace<T> fa(s_n, dtrdz), fb(s_1, dtrdz);
+    const T ca = s_k * u_k - s_n * d_k, cb = s_2 * u_2 - s_1 * d_2;
+#pragma unroll
+    for (int g = 0; g < N; ++g) {
+      // one field after the other: with the four chains interleaved the
+      // temporaries take the third wave per SIMD (225 VGPRs against 168)
+      if (g) __builtin_amdgcn_sched_barrier(0);
+      const T f1n = last ? T(0) : fa.flux(xm[g], x0[g], x1[g], x2[g]);
+      const T w1 = x0[g] - f1[g] * u_k + f1n * d_k + ca * x0[g];      // wz1(k)
+      if constexpr (emit) {
+        // y0, y1, w1 = wz1(k-2), wz1(k-1), wz1(k)
+        const T f2n = fb.flux(ym[g], y0[g], y1[g], w1);
+        *(T *)((char *)po[g] + ot) = y0[g] - f2[g] * u_2 + f2n * d_2 + cb * y0[g];
+        f2[g] = f2n;
+      }
+      po[g] += P;
+      f1[g] = f1n;
+      xm[g] = x0[g];
+      x0[g] = x1[g];
+      x1[g] = x2[g];
+      if constexpr (!last) x2[g] = x3[g];
+      ym[g] = y0[g];
+      y0[g] = y1[g];
+      y1[g] = w1;
+    }
+    s_2 = s_1;
+    s_1 = s_k;
+    s_k = s_n;
+    s_n = T(ns);
+    u_2 = u_1;
+    u_1 = u_k;
+    u_k = T(nu);
+    d_2 = d_1;
+    d_1 = d_k;
+    d_k = T(nd);
+  };
+  level(1, std::false_type{}, std::false_type{});
+  level(2, std::false_type{}, std::false_type{});
+  // the second half step's first face has x(0) = x(1)
+#pragma unroll
+  for (int g = 0; g < N; ++g) ym[g] = y0[g];
+  for (int k = 3; k < kz; ++k) level(k, std::true_type{}, std::false_type{});
+  level(kz, std::true_type{}, std::true_type{});
+  // wz2(kz-1) and wz2(kz): y0, y1 = wz1(kz-1), wz1(kz); s_k = s(kz+1)
+  const WafFace<T> fb(s_1, dtrdz);
+  const T cb = s_2 * u_2 - s_1 * d_2, cc = s_1 * u_1 - s_k * d_1;
+#pragma unroll
+  for (int g = 0; g < N; ++g) {
+    const T f2n = fb.flux(ym[g], y0[g], y1[g], y1[g]);
+    *(T *)((char *)po[g] + ot) = y0[g] - f2[g] * u_2 + f2n * d_2 + cb * y0[g];
+    *(T *)((char *)(po[g] + P) + ot) = y1[g] - f2n * u_1 + T(0) * d_1 + cc * y1[g];
+  }
+}
+
 template <typename T, typename S, int G>
 __device__ __forceinline__ void WafVertical<T, S, G>::run(const WafVertical &args_, int bx, int by,
                                                           int bz) {
   const Dims d = args_.d;
-  const AdvPtrs<T> &ap = args_.ap;
-  const S *__restrict__ s = args_.s;
-  const S *__restrict__ zrfmu = args_.zrfmu;
-  const S *__restrict__ zrfmd = args_.zrfmd;
-  const double dtrdz_ = args_.dtrdz_;
-
   const int j = 1 + bx * TJ + threadIdx.x;
   const int i = 1 + by * TI + threadIdx.y;
-  const int f0 = (int)bz * G;
-  const int ng = args_.nf - f0 < G ? args_.nf - f0 : G;
   if (j > d.je2 || i > d.ie2) return;
-  const T dtrdz = T(dtrdz_);
-  const int kz = d.kz;
-  const long long P = d.plane;
-  const long long c1 = d.at(j, i, 1);
-  const S *__restrict__ ps = s + c1;
-  const S *__restrict__ pu = zrfmu + c1;
-  const S *__restrict__ pd = zrfmd + c1;
-  const T *px[G];
-  T *po[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const int f = f0 + (g < ng ? g : 0);
-    px[g] = ap.src[f] + c1;
-    po[g] = ap.dst[f] + c1;
-  }
-  // per field: first half step window x(max(k-1,1)), x(k), x(k+1),
-  // x(min(k+2,kz)); wfw1 on the top face of level k; wz1 history; wfw2
-  T a_m1[G], a_0[G], a_1[G], a_2[G], f1[G], h1[G], h2[G], h3[G], f2[G];
-  const long long k3 = (long long)((3 <= kz ? 3 : kz) - 1) * P;
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    if (g < ng) {
-      a_m1[g] = px[g][0];
-      a_0[g] = a_m1[g];
-      a_1[g] = px[g][P];
-      a_2[g] = px[g][k3];
-    }
-    f1[g] = T(0);
-    h1[g] = h2[g] = h3[g] = T(0);
-    f2[g] = T(0);
-  }
-  T s_k = T(ps[0]);
-  T sm1 = T(0), sm2 = T(0);              // s(k-1), s(k-2)
-  T um1 = T(0), um2 = T(0), dm1 = T(0), dm2 = T(0);
-  // s(k+1), zrfmu(k), zrfmd(k) of the next level are requested a level
-  // ahead, before this level's stores (a load issued after a store would
-  // wait for the store as well)
-  S nx_s = ps[P], nx_u = pu[0], nx_d = pd[0];
-  for (int k = 1; k <= kz; ++k) {
-    const long long o = (long long)(k - 1) * P;
-    const T s_kp1 = T(nx_s);
-    const T zu = T(nx_u), zd = T(nx_d);
-    {
-      const long long on = k < kz ? o + P : o;   // level k + 1, clamped
-      nx_s = ps[on + P];
-      nx_u = pu[on];
-      nx_d = pd[on];
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      if (g < ng) {
-        const T f1n = (k < kz) ? waf_vflux(s_kp1, dtrdz, a_m1[g], a_0[g], a_1[g], a_2[g]) : T(0);
-        const T zdv = (s_k * zu - s_kp1 * zd) * a_0[g];
-        const T w1 = a_0[g] - f1[g] * zu + f1n * zd + zdv;     // wz1(k)
-        f1[g] = f1n;
-        {
-          const T t = a_2[g];
-          a_m1[g] = a_0[g];
-          a_0[g] = a_1[g];
-          a_1[g] = t;
-          a_2[g] = (k + 3 <= kz) ? px[g][(long long)(k + 2) * P] : t;
-        }
-        if (k >= 3) {                      // emit wz2(k-2)
-          const int kp = k - 2;
-          const T ym1 = (kp == 1) ? h2[g] : h3[g];
-          const T y0 = h2[g], y1 = h1[g], y2 = w1;
-          const T f2n = waf_vflux(sm1, dtrdz, ym1, y0, y1, y2);
-          const T zdv2 = (sm2 * um2 - sm1 * dm2) * y0;
-          po[g][(long long)(kp - 1) * P] = y0 - f2[g] * um2 + f2n * dm2 + zdv2;
-          f2[g] = f2n;
-        }
-        h3[g] = h2[g];
-        h2[g] = h1[g];
-        h1[g] = w1;
-      }
-    }
-    sm2 = sm1;
-    sm1 = s_k;
-    s_k = s_kp1;
-    um2 = um1;
-    um1 = zu;
-    dm2 = dm1;
-    dm1 = zd;
-  }
-  // flush wz2(kz-1) and wz2(kz): wz1 history is (h3, h2, h1) =
-  // (wz1(kz-2), wz1(kz-1), wz1(kz)); metrics of kz-1 in (sm2, um2, dm2), of
-  // kz in (sm1, um1, dm1); s(kz+1) in s_k
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    if (g < ng) {
-      {
-        const int kp = kz - 1;
-        const T ym1 = (kp == 1) ? h2[g] : h3[g];
-        const T y0 = h2[g], y1 = h1[g], y2 = h1[g];
-        const T f2n = waf_vflux(sm1, dtrdz, ym1, y0, y1, y2);   // s(kz)
-        const T zdv2 = (sm2 * um2 - sm1 * dm2) * y0;
-        po[g][(long long)(kp - 1) * P] = y0 - f2[g] * um2 + f2n * dm2 + zdv2;
-        f2[g] = f2n;
-      }
-      {
-        const T y0 = h1[g];                  // wz1(kz)
-        const T f2n = T(0);                  // wfw2(kz+1)
-        const T zdv2 = (sm1 * um1 - s_k * dm1) * y0;
-        po[g][(long long)(kz - 1) * P] = y0 - f2[g] * um1 + f2n * dm1 + zdv2;
-      }
-    }
+  // nf = ngroups * base + rest: the first `rest` groups take one field more
+  const int base = args_.nf / args_.ngroups, rest = args_.nf - base * args_.ngroups;
+  const int n = base + (bz < rest ? 1 : 0), f0 = bz * base + (bz < rest ? bz : rest);
+  const T dtrdz = T(args_.dtrdz_);
+  auto col = [&](auto c) {
+    if constexpr (decltype(c)::value <= G)
+      waf_column<decltype(c)::value, T, S>(d, args_.ap, args_.s, args_.zrfmu, args_.zrfmd, dtrdz,
+                                           f0, j, i);
+  };
+  switch (n) {
+    case 1: col(std::integral_constant<int, 1>{}); break;
+    case 2: col(std::integral_constant<int, 2>{}); break;
+    case 3: col(std::integral_constant<int, 3>{}); break;
+    default: col(std::integral_constant<int, 4>{}); break;
   }
 }
 
@@ -3174,22 +3248,22 @@ static int waf_vertical(mlc_handle *h, const Dims &d, const AdvPtrs<R> &vb, int 
   if constexpr (sizeof(R) == 4) {
     if (np && (h->tune.mixed_merge & 1)) {
       // float and double batches in one launch
-      constexpr int GD = 2;
+      constexpr int GD = G < 2 ? G : 2;
       using WafVM = WafVerticalMixed<R, G, GD>;
       const int ngf = (nb + G - 1) / G, ngd = (np + GD - 1) / GD;
       const WafVM a{WafVertical<float, R, G>{d, vb, h->s.as<R>(), h->zrfmu.as<R>(),
-                                             h->zrfmd.as<R>(), dtrdz, nb},
+                                             h->zrfmd.as<R>(), dtrdz, nb, ngf},
                     WafVertical<double, R, GD>{d, vp, h->s.as<R>(), h->zrfmu.as<R>(),
-                                               h->zrfmd.as<R>(), dtrdz, np},
+                                               h->zrfmd.as<R>(), dtrdz, np, ngd},
                     ngf};
       return emit(h, K_WAF_V, grid_cross(d, ngf + ngd), kBlock, 0, a);
     }
   }
   MLC_EMIT(K_WAF_V, WafVRR, grid_cross(d, (nb + G - 1) / G), kBlock, 0, d, vb,
-           h->s.as<R>(), h->zrfmu.as<R>(), h->zrfmd.as<R>(), dtrdz, nb);
+           h->s.as<R>(), h->zrfmu.as<R>(), h->zrfmd.as<R>(), dtrdz, nb, (nb + G - 1) / G);
   if (np)
     MLC_EMIT(K_WAF_V, WafVDR, grid_cross(d, (np + G - 1) / G), kBlock, 0, d, vp,
-             h->s.as<R>(), h->zrfmu.as<R>(), h->zrfmd.as<R>(), dtrdz, np);
+             h->s.as<R>(), h->zrfmu.as<R>(), h->zrfmd.as<R>(), dtrdz, np, (np + G - 1) / G);
   return MLC_OK;
 }
 
