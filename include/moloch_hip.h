@@ -212,14 +212,15 @@ int mlc_kernel_stats(mlc_handle *h, int slot, long long *launches,
 /* Launch-shape variants of a stage.  Every variant of a stage gives
  * bit-identical results; their speed depends on the domain shape.  No
  * reference counterpart (a GPU launch choice). */
-#define MLC_VAR_WAF_H 0       /* horizontal WAF: 0 row-streaming, 1 LDS tile (default) */
-#define MLC_VAR_WAF_ROWS 1    /* row-streaming WAF: i rows per wavefront, 4..256 (16) */
-#define MLC_VAR_WAF_GROUP 2   /* row-streaming WAF: fields per lane, 2 or 4 (4) */
+#define MLC_VAR_WAF_H 0       /* horizontal WAF: 0 row-streaming (default), 1 LDS tile */
+#define MLC_VAR_WAF_ROWS 1    /* row-streaming WAF: i rows per wavefront, 4..256 (by domain size) */
+#define MLC_VAR_WAF_GROUP 2   /* row-streaming WAF: fields per lane, 2 or 4 (by domain size) */
 #define MLC_VAR_LEVEL_CHUNK 3 /* divergence (and momentum, unless MLC_VAR_MOM_CHUNK is set):
                                  levels per thread, 1..kz (8) */
 #define MLC_VAR_COLUMN 4      /* column solve: 0 LDS three-phase, 1 streamed, 2 LDS with
                                  level chunks in registers (default; kz > 64 runs 0) */
-#define MLC_VAR_WAFV_GROUP 5  /* vertical WAF: fields per thread, 1, 2 or 4 (4) */
+#define MLC_VAR_WAFV_GROUP 5  /* vertical WAF: fields per thread, 1, 2 or 4 (by domain
+                                 size) */
 #define MLC_VAR_XCD_MAP 6     /* single-domain launches: 1 XCD-contiguous tile order (default), 0 plain */
 #define MLC_VAR_WAF_TILE 7    /* LDS-tile WAF: output rows per tile, 4 or 8 (default 8 in FP64, 4 mixed) */
 #define MLC_VAR_WAF_HGROUP 8  /* LDS-tile WAF: fields per block, 0 = the whole batch (default) */

@@ -549,6 +549,88 @@ static int build_bdy_tables(mlc_handle *h) {
   return MLC_OK;
 }
 
+// Fields per thread of the vertical WAF for nf fields on cross columns that
+// make `waves` wavefronts.  A SIMD runs its waves' levels one after the
+// other, and a level costs about 0.7 of a field on top of the fields (s and
+// the metric ratios), so the cost is the waves of the fullest of the chip's
+// 1024 SIMDs times (fields per wave + 0.7): few fields per wave where the
+// domain leaves SIMDs idle or unevenly filled, four where it fills them.
+// Measured, us per call at 4 / 2 / 1: 64x64x23 20.2 / 16.2 / 13.8,
+// 151x127x35 57 / 47 / 53, 500x100x60 144 / 128 / 162, 256x256x41 109 / 128 / 145.
+static int wafv_rule(long long waves, int nf) {
+  int best = 4;
+  double cost = 0.0;
+  for (int g = 4; g >= 1; g /= 2) {
+    const int groups = (nf + g - 1) / g;
+    const double c = (double)((waves * groups + 1023) / 1024) * ((double)nf / groups + 0.7);
+    if (g == 4 || c < cost) {
+      best = g;
+      cost = c;
+    }
+  }
+  return best;
+}
+
+// Rows per wave and fields per lane of the row-streaming horizontal WAF.  A
+// wave of r rows and g fields costs about (r + 2)(g + 1.2): two rows of start
+// (the window's loads and one face), and a row's coefficients weigh a little
+// more than a field.  Domains whose shortest chunks make fewer than two waves
+// per SIMD take the shape with the lowest cost times waves of the fullest
+// SIMD (a float wave leaves its SIMD idle about half the time, so a second
+// one costs half).  Larger domains take four fields and the longest chunk that
+// still leaves 12000 waves, an even load to the end of the launch: measured at
+// 256x256x41, us per call at 8 / 12 / 16 / 24 / 32 / 64 rows: FP64 216 / 214 /
+// 215 / 222 / 225 / 255, mixed 67 / 70 / 70 / 74 / 80 / 99; 151x127x35 at 4 /
+// 8 / 12: 56 / 58 / 62; 64x64x23 at 4 x 2, 6 x 2, 4 x 4, 8 x 4 (rows x
+// fields): 11.1 / 9.2 / 9.6 / 13.4.
+static void rows_rule(mlc_handle *const *h, int n, int *rows, int *group) {
+  const bool mixed = h[0]->mixed;
+  auto waves = [&](int r, int g) {
+    long long w = 0;
+    for (int m = 0; m < n; ++m) {
+      const Dims &d = h[m]->d;
+      const int nf = h[m]->nadvf - (mixed ? 2 : 0);
+      w += (long long)wr_tiles(d) * ((d.ie2 + r - 1) / r) * ((nf + g - 1) / g) * d.kz;
+    }
+    return w;
+  };
+  *group = 4;
+  *rows = 4;
+  if (waves(4, 4) <= 2048) {
+    double best = 0.0;
+    for (int g : {4, 2})
+      for (int r : {4, 6, 8}) {
+        const double load = (double)waves(r, g) / 1024.0;
+        const double fill = load <= 1.0 ? 1.0 : (mixed ? 0.5 * (1.0 + load) : std::ceil(load));
+        const double c = fill * (r + 2.0) * (g + 1.2);
+        if (best == 0.0 || c < best) {
+          best = c;
+          *rows = r;
+          *group = g;
+        }
+      }
+    return;
+  }
+  for (int r : {6, 8, 12, 16})
+    if (waves(r, 4) >= 12000) *rows = r;
+}
+
+void waf_shapes(mlc_handle *const *h, int n) {
+  long long waves = 0;
+  int nf = 0, rows = 0, group = 0;
+  for (int m = 0; m < n; ++m) {
+    waves += column_waves(h[m]->d);
+    nf = h[m]->nadvf > nf ? h[m]->nadvf : nf;
+  }
+  const int wafv = wafv_rule(waves, nf);
+  rows_rule(h, n, &rows, &group);
+  for (int m = 0; m < n; ++m) {
+    h[m]->tune.wafv_group = wafv;
+    h[m]->tune.waf_rows = rows;
+    h[m]->tune.waf_group = group;
+  }
+}
+
 int create_handle(const mlc_grid_desc *g, hipStream_t shared, mlc_handle **out) {
   if (!g || !out) return fail(MLC_E_ARG, "null argument");
   *out = nullptr;
@@ -595,7 +677,7 @@ int create_handle(const mlc_grid_desc *g, hipStream_t shared, mlc_handle **out) 
     h->s_tr0 = h->nslots;
     for (int n = 0; n < g->ntr; ++n) h->adv_list[h->nadvf++] = h->nslots++;
   }
-  h->tune.wafv_group = wafv_rule(column_waves(h->d), h->nadvf);
+  waf_shapes(&h, 1);
   h->h_mx.assign((size_t)h->d.plane, 0.0);
   h->h_mu.assign((size_t)h->d.plane, 0.0);
   h->h_mv.assign((size_t)h->d.plane, 0.0);

@@ -262,13 +262,7 @@ int mlc_batch_create(const mlc_grid_desc *descs, int n, mlc_batch **out) {
     b->npoints += mlc_npoints(h);
   }
   // the members' launches are merged: one choice, by their common grid
-  long long waves = 0;
-  int nf = 0;
-  for (const mlc_handle *h : b->all) {
-    waves += column_waves(h->d);
-    nf = h->nadvf > nf ? h->nadvf : nf;
-  }
-  for (mlc_handle *h : b->all) h->tune.wafv_group = wafv_rule(waves, nf);
+  waf_shapes(b->all.data(), n);
   *out = b;
   return MLC_OK;
 }

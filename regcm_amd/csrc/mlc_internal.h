@@ -172,31 +172,18 @@ struct ZMet {
   }
 };
 
-// Fields per thread of the vertical WAF for nf fields on cross columns that
-// make `waves` wavefronts.  A SIMD runs its waves' levels one after the
-// other, and a level costs about 0.7 of a field on top of the fields (s and
-// the metric ratios), so the cost is the waves of the fullest of the chip's
-// 1024 SIMDs times (fields per wave + 0.7): few fields per wave where the
-// domain leaves SIMDs idle or unevenly filled, four where it fills them.
-// Measured, us per call at 4 / 2 / 1: 64x64x23 20.2 / 16.2 / 13.8,
-// 151x127x35 57 / 47 / 53, 500x100x60 144 / 128 / 162, 256x256x41 109 / 128 / 145.
-inline int wafv_rule(long long waves, int nf) {
-  int best = 4;
-  double cost = 0.0;
-  for (int g = 4; g >= 1; g /= 2) {
-    const int groups = (nf + g - 1) / g;
-    const double c = (double)((waves * groups + 1023) / 1024) * ((double)nf / groups + 0.7);
-    if (g == 4 || c < cost) {
-      best = g;
-      cost = c;
-    }
-  }
-  return best;
-}
-
 // Wavefronts of 64 x 1 columns that cover a domain's cross points.
 inline long long column_waves(const Dims &d) {
   return (long long)((d.je2 + 63) / 64) * ((d.ie2 + 3) / 4) * 4;
+}
+
+// Row-streaming horizontal WAF: output j points of a wavefront with halos on
+// both sides, and its j tiles on a domain (a bounded domain's first tile
+// starts at lane 0 and its last ends at lane 63).
+constexpr int kWrOut = 60;
+inline int wr_tiles(const Dims &d) {
+  if (d.crm) return (d.jx + kWrOut - 1) / kWrOut;
+  return d.je2 <= 64 ? 1 : 1 + (d.je2 - 64 + kWrOut - 1) / kWrOut;
 }
 
 // Kernel slots for per-kernel timing.
@@ -309,14 +296,14 @@ struct mlc_handle {
 
   // launch-shape choices (autotuned per domain shape)
   struct Tune {
-    int waf_h = 1;               // horizontal WAF: 0 row-streaming, 1 LDS tile
-    int waf_rows = 16;           // row-streaming WAF: i rows per wavefront
-    int waf_group = 4;           // row-streaming WAF: fields per lane (2 or 4)
+    int waf_h = 0;               // horizontal WAF: 0 row-streaming, 1 LDS tile
+    int waf_rows = 16;           // row-streaming WAF: i rows per wavefront (waf_shapes)
+    int waf_group = 4;           // row-streaming WAF: fields per lane (2 or 4; waf_shapes)
     int level_chunk = 8;         // divergence/momentum: levels per thread
     int mom_chunk = 0;           // momentum, if not 0: levels per thread
     int stag_chunk = 1;          // staggering passes: levels per thread
     int column = 2;              // column solve: 0 LDS three-phase, 1 streamed, 2 chunked
-    int wafv_group = 4;          // vertical WAF: fields per thread (1, 2 or 4; wafv_rule)
+    int wafv_group = 4;          // vertical WAF: fields per thread (1, 2 or 4; waf_shapes)
     int xcd_map = 1;             // XCD-contiguous tile order of single-domain launches
     int waf_tile = 4;            // LDS-tile WAF: output rows per tile (4 or 8; FP64 starts at 8)
     int waf_hgroup = 0;          // LDS-tile WAF: fields per block (0 = the whole batch)
@@ -337,6 +324,10 @@ struct mlc_handle {
 };
 
 namespace mlc {
+
+// Sets the WAF launch shapes of handles whose stages run in common launches
+// (one handle, or a batch's members) from their sizes.
+void waf_shapes(mlc_handle *const *h, int n);
 
 // Error reporting (thread-local message).
 int fail(int code, const std::string &msg);

@@ -20,6 +20,7 @@
 #include <mutex>
 #include <string>
 #include <type_traits>
+#include <utility>
 
 #include <hip/hip_ext.h>
 
@@ -1726,223 +1727,313 @@ struct WafHorizontalMixed {
 
 // ---------------------------------------------------------------------------
 // The same meridional + zonal passes in row-streaming form.  A wavefront
-// owns 64 consecutive j points of one level (kWrOut outputs and 2 halo
-// points each side) and marches down a chunk of kWrRows i rows.  Each lane
-// keeps the last four rows of wz in registers, so the meridional flux needs
-// no other lane; the zonal neighbours of p0 and of the zonal flux come from
-// the other lanes of the wavefront by shuffles.  No LDS, no barriers.  A
-// lane handles a group of up to kWrG fields, so the field-independent
-// coefficients of a point are formed once per group.  Every value is formed
-// with the operations and operand order of WafHorizontal.
-constexpr int kWrOut = 60;     // output j points per wavefront
-constexpr int kWrWaves = 4;    // wavefronts (i chunks) per block
+// owns 64 consecutive j points of one level and marches down a chunk of i
+// rows with up to four fields.  Each lane keeps the rows i .. i+2 of wz in
+// registers, so the meridional flux needs no other lane; the zonal neighbours
+// of p0 and of the zonal flux come from the lanes next to it by DPP wave
+// shifts.  No LDS, no barriers.  The field-independent coefficients of a row
+// are formed once for the wave's fields, and a row's operands are requested a
+// row ahead.  Every value is formed with the operations and operand order of
+// WafHorizontal; a face's limiter ratio is a ratio of first differences, each
+// difference formed once and passed on.
+//
+// What bounds it: about evenly the issue of its instructions (119 per field
+// and point, of which 20 move windows and neighbours) and its 3F + 4 arrays.
+// The LDS-tile form spends a third of its lanes on partly filled passes over
+// halos and waits at four barriers per field.  Per call, tile form -> this:
+// 24x20x10 22.2 -> 8.2 us, 64x64x23 19.3 -> 9.6, 151x127x35 89 -> 56,
+// 500x100x60 290 -> 234, 256x256x41 FP64 248 -> 212 (3.4 TB/s), mixed 2 x 96
+// -> 2 x 67 (Pi and theta_v, and the float fields), 512x512x41 mixed 2 x 367
+// -> 2 x 243.
+//
+// A wave's outputs: lanes 2 .. 61, and on a bounded domain also the lanes at
+// the west and east edge, which need no halo (the upwind clamps of
+// init_moloch make the west edge's outer difference zero and let the east
+// edge's stand in for its own neighbour).
+constexpr int kWrWaves = 4;    // wavefronts per block
 
-template <typename T>
-__device__ __forceinline__ T sel4(int o, T a0, T a1, T a2, T a3) {
-  return o == 0 ? a0 : (o == 1 ? a1 : (o == 2 ? a2 : a3));
+// The value of the next lane (lane 63: zero) and of the previous one (lane 0:
+// its own).
+__device__ __forceinline__ int lane_next(int x) {
+  return __builtin_amdgcn_mov_dpp(x, 0x130, 0xf, 0xf, true);          // wave_shl:1
+}
+__device__ __forceinline__ int lane_prev(int x) {
+  return __builtin_amdgcn_update_dpp(x, x, 0x138, 0xf, 0xf, false);   // wave_shr:1
+}
+__device__ __forceinline__ float lane_next(float x) {
+  return __int_as_float(lane_next(__float_as_int(x)));
+}
+__device__ __forceinline__ float lane_prev(float x) {
+  return __int_as_float(lane_prev(__float_as_int(x)));
+}
+__device__ __forceinline__ double lane_next(double x) {
+  return __hiloint2double(lane_next(__double2hiint(x)), lane_next(__double2loint(x)));
+}
+__device__ __forceinline__ double lane_prev(double x) {
+  return __hiloint2double(lane_prev(__double2hiint(x)), lane_prev(__double2loint(x)));
 }
 
-template <typename T, typename S, int kWrG>
+template <typename T, typename S, int PER, int ROT>
 struct WafRows {
   Dims d;
   AdvPtrs<T> ap;
   AdvPtrs<T> wzp;
   int nf;
-  int ngroups;
+  int ngroups;                 // near-equal groups of at most four fields
   int rows;                    // i rows per chunk
+  int nchunk, ntile;           // chunks along i, tiles along j
   const S *u, *v, *mu, *mv, *mx, *mx2, *rmu, *rmv, *rfmzu, *rfmzv, *fmz;
   double dtrdx_, dtrdy_;
-  int rotllr;
+  // the curvature terms of advection (:811-825) on fields 0 (ux) and 1 (vx)
+  int curv;
+  const S *tanrot;
+  double rdx_, dta_;
   static __device__ __forceinline__ void run(const WafRows &args_, int bx, int by, int bz);
 };
 
-template <typename T, typename S, int kWrG>
-__device__ __forceinline__ void WafRows<T, S, kWrG>::run(const WafRows &args_, int bx, int by, int bz) {
-  const Dims d = args_.d;
-  const int jce2 = d.jx - 1, ice2 = d.iy - 1;
-  const int jmin = 1, jmax = jce2, imin = 1, imax = ice2;
-  const int rows = args_.rows;
-  const int chunk = by * kWrWaves + (int)threadIdx.y;
-  const int i0 = 1 + chunk * rows;
-  if (i0 > ice2) return;                          // uniform per wavefront
-  const int i1 = i0 + rows - 1 < ice2 ? i0 + rows - 1 : ice2;
-  const int ngroups = args_.ngroups;
-  const int grp = bz % ngroups;
-  const int k = 1 + bz / ngroups;
-  const int f0 = grp * kWrG;
-  const int ng = args_.nf - f0 < kWrG ? args_.nf - f0 : kWrG;
+template <int N, typename T, typename S, int PER, int ROT>
+__device__ __forceinline__ void waf_rows_body(const WafRows<T, S, PER, ROT> &a, int f0, int tile,
+                                              int chunk, int k) {
+  const Dims d = a.d;
+  constexpr bool rotllr = ROT != 0;
   const int lane = threadIdx.x;
-  const int jj = bx * kWrOut - 1 + lane;          // j0 - 2 + lane, j0 = 1 + kWrOut*bx
-  const bool jin = jj >= 1 && jj <= jce2;
-  const bool jout = jin && lane >= 2 && lane < 2 + kWrOut;
-  const int jc = jin ? jj : 1;
-  const int rotllr = args_.rotllr;
-  const S dtrdx = S(args_.dtrdx_), dtrdy = S(args_.dtrdy_);
-  const long long pj = d.pj;
-  const S *__restrict__ u = args_.u;
-  const S *__restrict__ v = args_.v;
-  const S *__restrict__ mu = args_.mu;
-  const S *__restrict__ mv = args_.mv;
-  const S *__restrict__ mx = args_.mx;
-  const S *__restrict__ mx2 = args_.mx2;
-  const S *__restrict__ rmu = args_.rmu;
-  const S *__restrict__ rmv = args_.rmv;
-  const S *__restrict__ rfmzu = args_.rfmzu;
-  const S *__restrict__ rfmzv = args_.rfmzv;
-  const S *__restrict__ fmz = args_.fmz;
-  const T *wz[kWrG];
-  const T *pp[kWrG];
-  T *po[kWrG];
-#pragma unroll
-  for (int g = 0; g < kWrG; ++g) {
-    const int f = f0 + (g < ng ? g : 0);
-    wz[g] = args_.wzp.src[f];
-    pp[g] = args_.ap.src[f];
-    po[g] = args_.ap.dst[f];
+  const int je2 = d.je2, ie2 = d.ie2;
+  const int i0 = 1 + chunk * a.rows;
+  const int i1 = i0 + a.rows - 1 < ie2 ? i0 + a.rows - 1 : ie2;
+  const int ic1 = PER ? 1 : 2, ic2 = PER ? ie2 : ie2 - 1;
+  // this lane's column; past the domain a lane repeats the edge column (or,
+  // periodic, the partner column two past the edge)
+  int j, jc;
+  bool jout;
+  if (PER) {
+    j = tile * kWrOut - 1 + lane;
+    const int jl = j < je2 + 2 ? j : je2 + 2;
+    jc = jl < 1 ? jl + je2 : (jl > je2 ? jl - je2 : jl);
+    jout = lane >= 2 && lane < 2 + kWrOut && j <= je2;
+  } else {
+    j = tile * kWrOut + 1 + lane;
+    jc = j < je2 ? j : je2;
+    const int jlast = tile * kWrOut + 64;      // the column of lane 63
+    jout = (tile == 0 || lane >= 2) && (jlast >= je2 || lane < 62) && j <= je2;
   }
-  auto wz_row = [&](int g, int r) -> T {
-    return (jin && r >= 1 && r <= ice2) ? wz[g][d.at(jj, r, k)] : T(0);
+  const bool jend = !PER && j == je2;
+  const bool jint = PER ? true : (j >= 2 && j <= je2 - 1);
+  // byte offsets of a row for this lane; an array's level base is uniform
+  auto row = [&](int i) -> unsigned {
+    int r = i;
+    if (PER)
+      r = i < 1 ? i + ie2 : (i > ie2 ? i - ie2 : i);
+    else
+      r = i < 1 ? 1 : (i > ie2 ? ie2 : i);
+    return (unsigned)((r - 1) * d.pj + (jc - 1));
   };
-  // meridional flux through face ii from the window rows ii-2 .. ii+1
-  auto zpby = [&](int ii, S vv, S mvv, const T *W) -> T {
-    const S zamu = rotllr ? vv * dtrdy : vv * mvv * dtrdy;
-    T is;
-    int ih;
-    if (zamu > S(0)) {
-      is = T(1);
-      ih = ii - 1;
-    } else {
-      is = T(-1);
-      ih = ii + 1 < imax ? ii + 1 : imax;
-    }
-    const int ihm1 = ih - 1 > imin ? ih - 1 : imin;
-    const T wh = sel4(ih - (ii - 2), W[0], W[1], W[2], W[3]);
-    const T whm1 = sel4(ihm1 - (ii - 2), W[0], W[1], W[2], W[3]);
-    const T rr = flow_param(wh - whm1, W[2] - W[1]);
-    const T b = waf_b(rr);
-    const T zphi = is + T(zamu) * b - is * b;
-    return T(S(0.5) * vv) * ((T(1) + zphi) * W[1] + (T(1) - zphi) * W[2]);
+  auto ld = [](const auto *p, unsigned o) {
+    using X = typename std::remove_cv<typename std::remove_reference<decltype(*p)>::type>::type;
+    return *(const X *)((const char *)p + o * (unsigned)sizeof(X));
   };
-  auto face_v = [&](int ii, S *vv, S *mvv) {
-    const bool ok = jin && ii >= 2 && ii <= ice2;
-    *vv = ok ? v[d.at(jc, ii, k)] : S(0);
-    *mvv = ok ? mv[d.at2(jc, ii)] : S(0);
+  const long long lk = (long long)(k - 1) * d.plane;
+  const S *u = a.u + lk, *v = a.v + lk, *fmz = a.fmz + lk, *ru_ = a.rfmzu + lk;
+  // the meridional fluxes take rfmzv with ROTLLR, else rfmzu (:1004-1005)
+  const S *ry_ = rotllr ? a.rfmzv + lk : ru_;
+  const S *mxs = rotllr ? a.mx : a.mx2;
+  const T *wz[N], *pp[N];
+  T *po[N];
+#pragma unroll
+  for (int g = 0; g < N; ++g) {
+    wz[g] = a.wzp.src[f0 + g] + lk;
+    pp[g] = a.ap.src[f0 + g] + lk;
+    po[g] = a.ap.dst[f0 + g] + lk;
+  }
+  const S dtrdx = S(a.dtrdx_), dtrdy = S(a.dtrdy_);
+  const bool curv = N > 1 && a.curv && f0 == 0;
+
+  // the meridional face i: Courant number, 0.5 v
+  struct Face { T az, half; bool up; };
+  auto face_y = [&](S vv, S mvv) {
+    const S z = rotllr ? vv * dtrdy : vv * mvv * dtrdy;
+    return Face{T(fabs(z)), T(S(0.5) * vv), z > S(0)};
+  };
+  auto flux = [](const Face &fc, T prev, T here, T next, T lo, T hi) -> T {
+    const T b = waf_b(flow_param_sel(fc.up ? prev : next, here));
+    const T zphi = waf_phi(fc.az, b, fc.up);
+    return fc.half * ((T(1) + zphi) * lo + (T(1) - zphi) * hi);
   };
 
-  T W[kWrG][4], zprev[kWrG];
-  S v_i, mv_i;                                    // v, mv on face i
-  face_v(i0, &v_i, &mv_i);
+  // window of each field: wz(i), wz(i+1), wz(i+2); differences across the
+  // faces i and i+1; the flux through face i
+  T w0[N], w1[N], w2[N], dp[N], dc[N], fy[N];
+  // carried from row to row: v, rmv, ry and mv of row i
+  S v_i, rmv_i, ry_i, mv_i;
+  {
+    const unsigned om = row(i0 - 2), o1 = row(i0 - 1), o = row(i0), n = row(i0 + 1),
+                   n2 = row(i0 + 2);
+    T wm[N], wp[N];
 #pragma unroll
-  for (int g = 0; g < kWrG; ++g) {
-    if (g < ng) {
-      T W0[4] = {wz_row(g, i0 - 2), wz_row(g, i0 - 1), wz_row(g, i0), wz_row(g, i0 + 1)};
-      zprev[g] = (jin && i0 >= 2) ? zpby(i0, v_i, mv_i, W0) : T(0);
-      W[g][0] = W0[1];
-      W[g][1] = W0[2];
-      W[g][2] = W0[3];
-      W[g][3] = wz_row(g, i0 + 2);
+    for (int g = 0; g < N; ++g) {
+      wm[g] = ld(wz[g], om);
+      wp[g] = ld(wz[g], o1);
+      w0[g] = ld(wz[g], o);
+      w1[g] = ld(wz[g], n);
+      w2[g] = ld(wz[g], n2);
+    }
+    v_i = ld(v, o);
+    mv_i = ld(a.mv, o);
+    rmv_i = ld(a.rmv, o);
+    ry_i = ld(ry_, o);
+    const Face fc = face_y(v_i, mv_i);
+    const bool last = !PER && i0 >= ie2;       // face ie2: the upwind clamp
+#pragma unroll
+    for (int g = 0; g < N; ++g) {
+      const T dm = wp[g] - wm[g];
+      dp[g] = w0[g] - wp[g];
+      dc[g] = last ? dp[g] : w1[g] - w0[g];
+      fy[g] = flux(fc, dm, dp[g], dc[g], wp[g], w0[g]);
     }
   }
-  for (int i = i0; i <= i1; ++i) {
-    S v_n, mv_n;                                  // face i+1
-    face_v(i + 1, &v_n, &mv_n);
-    const bool row_in = i >= 2 && i <= ice2 - 1;
-    const long long c = d.at(jc, i, k), c2 = d.at2(jc, i);
-    // field-independent coefficients of p0 (row i) and of the zonal pass
-    S zrfmn = S(0), zrfms = S(0), cdv = S(0), mf = S(1);
-    S uu = S(0), zamu_u = S(0), is_u = S(0);
-    int oh = 0, ohm1 = 0;
-    if (jin && row_in) {
-      if (rotllr) {
-        const S zhxvtn = dtrdy * rmv[c2 + pj] * mx[c2];
-        const S zhxvts = dtrdy * rmv[c2] * mx[c2];
-        zrfmn = zhxvtn * fmz[c] * rfmzv[c + pj];
-        zrfms = zhxvts * fmz[c] * rfmzv[c];
-        cdv = v[c + pj] * zrfmn - v[c] * zrfms;
-      } else {
-        // rfmzu, not rfmzv, on the meridional fluxes (:1004-1005)
-        zrfmn = dtrdy * fmz[c] * rfmzu[c + pj];
-        zrfms = dtrdy * fmz[c] * rfmzu[c];
-        cdv = v[c + pj] * rmv[c2 + pj] * zrfmn - v[c] * rmv[c2] * zrfms;
-        mf = mx2[c2];
-      }
-      if (jj >= 2) {
-        uu = u[c];
-        zamu_u = uu * mu[c2] * dtrdx;
-        int jh;
-        if (zamu_u > S(0)) {
-          is_u = S(1);
-          jh = jj - 1;
-        } else {
-          is_u = S(-1);
-          jh = jj + 1 < jmax ? jj + 1 : jmax;
-        }
-        const int jhm1 = jh - 1 > jmin ? jh - 1 : jmin;
-        oh = jh - jj + 2;                         // offsets -2..+1 -> 0..3
-        ohm1 = jhm1 - jj + 2;
-      }
-    }
-    // coefficients of the final update (interior points of row i)
-    const bool o_int = jout && row_in && jj >= 2 && jj <= jce2 - 1;
-    S o_zrfmw = S(0), o_zrfme = S(0), o_cdv = S(0), o_mf = S(1);
-    if (o_int) {
-      if (rotllr) {
-        const S zcostx = dtrdx * mx[c2];
-        o_zrfmw = zcostx * fmz[c] * rfmzu[c];
-        o_zrfme = zcostx * fmz[c] * rfmzu[c + 1];
-        o_cdv = u[c + 1] * o_zrfme - u[c] * o_zrfmw;
-      } else {
-        o_zrfmw = dtrdx * fmz[c] * rfmzu[c];
-        o_zrfme = dtrdx * fmz[c] * rfmzu[c + 1];
-        o_cdv = u[c + 1] * rmu[c2 + 1] * o_zrfme - u[c] * rmu[c2] * o_zrfmw;
-        o_mf = mx2[c2];
-      }
-    }
+  // the operands of a row, requested a row ahead
+  struct Row {
+    S v_n, mv_n, rmv_n, ry_n, fz, uu, muu, rmuu, mxx, ruu;
+    T w3[N], pold[N];
+  };
+  auto request = [&](int i, Row &q) {
+    const unsigned o = row(i), w = row(i + 3);
+    // face i + 1: row iy of the staggered arrays on a bounded domain's last row
+    const unsigned n = PER ? row(i + 1) : (unsigned)(i * d.pj + (jc - 1));
 #pragma unroll
-    for (int g = 0; g < kWrG; ++g) {
-      if (g < ng) {
-        const T znext = (jin && i + 1 <= ice2) ? zpby(i + 1, v_n, mv_n, W[g]) : T(0);
-        const T pold = jin ? pp[g][c] : T(0);
-        T p0 = T(0);
-        if (jin && row_in) {
-          const T zdv = T(cdv) * pold;
-          const T x = zprev[g] * T(zrfms) - znext * T(zrfmn) + zdv;
-          // ROTLLR has no mx2 factor; mf = 1 there and 1*x == x exactly
-          p0 = W[g][1] + T(mf) * x;
-        }
-        // zonal flux through face jj from p0 at jj-2 .. jj+1
-        const T pm2 = __shfl(p0, lane >= 2 ? lane - 2 : 0);
-        const T pm1 = __shfl(p0, lane >= 1 ? lane - 1 : 0);
-        const T pp1 = __shfl(p0, lane <= 62 ? lane + 1 : 63);
-        T zpbw = T(0);
-        if (jin && row_in && jj >= 2) {
-          const T rr = flow_param(sel4(oh, pm2, pm1, p0, pp1) - sel4(ohm1, pm2, pm1, p0, pp1),
-                                  p0 - pm1);
-          const T b = waf_b(rr);
-          const T zphi = T(is_u) + T(zamu_u) * b - T(is_u) * b;
-          zpbw = T(S(0.5) * uu) * ((T(1) + zphi) * pm1 + (T(1) - zphi) * p0);
-        }
-        const T ze = __shfl(zpbw, lane <= 62 ? lane + 1 : 63);
-        if (jout) {
-          T val = pold;
-          if (o_int) {
-            const T zdv = T(o_cdv) * pold;
-            if (rotllr)
-              val = p0 + zpbw * T(o_zrfmw) - ze * T(o_zrfme) + zdv;
-            else
-              val = p0 + T(o_mf) * (zpbw * T(o_zrfmw) - ze * T(o_zrfme) + zdv);
-          }
-          po[g][c] = val;
-        }
-        zprev[g] = znext;
-        W[g][0] = W[g][1];
-        W[g][1] = W[g][2];
-        W[g][2] = W[g][3];
-        W[g][3] = wz_row(g, i + 3);
-      }
+    for (int g = 0; g < N; ++g) {
+      q.w3[g] = ld(wz[g], w);
+      q.pold[g] = ld(pp[g], o);
     }
-    v_i = v_n;
-    mv_i = mv_n;
+    q.v_n = ld(v, n);
+    q.mv_n = ld(a.mv, n);
+    q.rmv_n = ld(a.rmv, n);
+    q.ry_n = ld(ry_, n);
+    q.fz = ld(fmz, o);
+    q.uu = ld(u, o);
+    q.muu = ld(a.mu, o);
+    q.rmuu = ld(a.rmu, o);
+    q.mxx = ld(mxs, o);
+    q.ruu = rotllr ? ld(ru_, o) : S(0);
+  };
+  S mv_s = ld(a.mv, row(i0 - 1));              // mv of row i - 1 (curvature)
+  Row ra, rb;
+  request(i0, ra);
+  // row i from its operands q; row i + 1's are requested into nx first
+  auto do_row = [&](int i, const Row &q, Row &nx) __attribute__((always_inline)) {
+    if (i < i1) request(i + 1, nx);
+    const bool row_in = PER || (i >= ic1 && i <= ic2);
+    const bool keep = !(row_in && jint);
+    const unsigned o = row(i);
+    // coefficients of the row, with the reference's operand order
+    const S ruu = rotllr ? q.ruu : ry_i;
+    const S rue = lane_next(ruu);
+    S zn, zs, cdv, zw, ze, odv, mf = S(1);
+    if constexpr (rotllr) {
+      zn = dtrdy * q.rmv_n * q.mxx * q.fz * q.ry_n;
+      zs = dtrdy * rmv_i * q.mxx * q.fz * ry_i;
+      cdv = q.v_n * zn - v_i * zs;
+      const S zcostx = dtrdx * q.mxx;
+      zw = zcostx * q.fz * ruu;
+      ze = zcostx * q.fz * rue;
+      odv = lane_next(q.uu) * ze - q.uu * zw;
+    } else {
+      zn = dtrdy * q.fz * q.ry_n;
+      zs = dtrdy * q.fz * ry_i;
+      cdv = q.v_n * q.rmv_n * zn - v_i * rmv_i * zs;
+      mf = q.mxx;
+      zw = dtrdx * q.fz * ruu;
+      ze = dtrdx * q.fz * rue;
+      const S ur = q.uu * q.rmuu;
+      odv = lane_next(ur) * ze - ur * zw;
+    }
+    const Face fn = face_y(q.v_n, q.mv_n);
+    const S zx = q.uu * q.muu * dtrdx;
+    const Face fx{T(fabs(zx)), T(S(0.5) * q.uu), zx > S(0)};
+    const bool last = !PER && i + 1 >= ie2;    // face ie2: the upwind clamp
+    T first = T(0);
+#pragma unroll
+    for (int g = 0; g < N; ++g) {
+      // one field after the other, for the registers (165 at four fields, three
+      // waves per SIMD)
+      if (g) __builtin_amdgcn_sched_barrier(0);
+      const T dn = last ? dc[g] : w2[g] - w1[g];
+      const T fyn = flux(fn, dp[g], dc[g], dn, w0[g], w1[g]);
+      const T pold = q.pold[g];
+      T p0 = fy[g] * T(zs) - fyn * T(zn) + T(cdv) * pold;
+      if constexpr (!rotllr) p0 = T(mf) * p0;
+      p0 = w0[g] + p0;
+      const T pm = lane_prev(p0);
+      const T df = p0 - pm;
+      const T dl = lane_prev(df);
+      T dr = lane_next(df);
+      dr = jend ? df : dr;
+      const T f = flux(fx, dl, df, dr, pm, p0);
+      const T fe = lane_next(f);
+      T val;
+      if constexpr (rotllr)
+        val = p0 + f * T(zw) - fe * T(ze) + T(odv) * pold;
+      else
+        val = p0 + T(mf) * (f * T(zw) - fe * T(ze) + T(odv) * pold);
+      val = keep ? pold : val;
+      if (N > 1 && g == 0) {
+        first = val;                           // stored with field 1
+      } else {
+        if (g == 1) {
+          if (curv) {
+            S tanx, tany;
+            if constexpr (rotllr) {
+              tanx = tany = ld(a.tanrot, o);
+            } else {
+              tanx = (lane_prev(q.muu) - q.muu) * S(a.rdx_);
+              tany = (mv_s - mv_i) * S(a.rdx_);
+            }
+            const T x = first + first * val * T(tanx) * T(S(a.dta_));
+            const T y = val - x * x * T(tany) * T(S(a.dta_));
+            first = keep ? first : x;
+            val = keep ? val : y;
+          }
+          if (jout) *(T *)((char *)po[0] + o * (unsigned)sizeof(T)) = first;
+        }
+        if (jout) *(T *)((char *)po[g] + o * (unsigned)sizeof(T)) = val;
+      }
+      fy[g] = fyn;
+      dp[g] = dc[g];
+      dc[g] = dn;
+      w0[g] = w1[g];
+      w1[g] = w2[g];
+      w2[g] = q.w3[g];
+    }
+    mv_s = mv_i;
+    v_i = q.v_n;
+    mv_i = q.mv_n;
+    rmv_i = q.rmv_n;
+    ry_i = q.ry_n;
+  };
+  for (int i = i0;;) {
+    do_row(i, ra, rb);
+    if (++i > i1) break;
+    do_row(i, rb, ra);
+    if (++i > i1) break;
+  }
+}
+
+template <typename T, typename S, int PER, int ROT>
+__device__ __forceinline__ void WafRows<T, S, PER, ROT>::run(const WafRows &a, int bx, int by, int bz) {
+  // one wave per (tile, group, chunk, level), tiles fastest: the wave index is
+  // uniform, and the groups of a chunk, which share its coefficients, and the
+  // tiles beside it, whose halos overlap, run next to it
+  const int id = __builtin_amdgcn_readfirstlane(bx * kWrWaves + (int)threadIdx.y);
+  const int tile = id % a.ntile, r1 = id / a.ntile;
+  const int grp = r1 % a.ngroups, r2 = r1 / a.ngroups;
+  const int chunk = r2 % a.nchunk, k = 1 + r2 / a.nchunk;
+  if (k > a.d.kz) return;
+  const int base = a.nf / a.ngroups, rest = a.nf - base * a.ngroups;
+  const int n = base + (grp < rest ? 1 : 0), f0 = grp * base + (grp < rest ? grp : rest);
+  switch (n) {
+    case 1: waf_rows_body<1, T, S, PER, ROT>(a, f0, tile, chunk, k); break;
+    case 2: waf_rows_body<2, T, S, PER, ROT>(a, f0, tile, chunk, k); break;
+    case 3: waf_rows_body<3, T, S, PER, ROT>(a, f0, tile, chunk, k); break;
+    default: waf_rows_body<4, T, S, PER, ROT>(a, f0, tile, chunk, k); break;
   }
 }
 
@@ -3340,30 +3431,44 @@ static int waf_tile(mlc_handle *h, const Dims &d, const AdvPtrs<R> &hb,
   return MLC_OK;
 }
 
-template <typename R, int G>
-static int waf_rows(mlc_handle *h, const Dims &d, const AdvPtrs<R> &hb,
-                    const AdvPtrs<R> &wzb, int nb, const AdvPtrs<double> &hp,
-                    const AdvPtrs<double> &wzp, int np, double dtrdx, double dtrdy) {
-  using WafRRR = WafRows<R, R, G>;
-  using WafRDR = WafRows<double, R, G>;
-  const int rot = h->g.lrotllr;
-  const int rows = h->tune.waf_rows;
-  const int ice2 = d.iy - 1, jce2 = d.jx - 1;
-  const int nchunk = (ice2 + rows - 1) / rows;
-  const unsigned gx = (unsigned)((jce2 + kWrOut - 1) / kWrOut);
-  const unsigned gy = (unsigned)((nchunk + kWrWaves - 1) / kWrWaves);
+template <typename R, int PER, int ROT>
+static int waf_rows(mlc_handle *h, const Dims &d, AdvPtrs<R> hb, AdvPtrs<R> wzb, int nb,
+                    const AdvPtrs<double> &hp, const AdvPtrs<double> &wzp, int np, double dtrdx,
+                    double dtrdy, int cux, int cvx, bool *curv) {
+  using WafRRR = WafRows<R, R, PER, ROT>;
+  using WafRDR = WafRows<double, R, PER, ROT>;
+  const int rows = h->tune.waf_rows, G = h->tune.waf_group;
+  const int nchunk = (d.ie2 + rows - 1) / rows, ntile = wr_tiles(d);
   const dim3 rblk(64, kWrWaves, 1);
-  const int ngb = (nb + G - 1) / G;
-  MLC_EMIT(K_WAF_H, WafRRR, dim3(gx, gy, (unsigned)(d.kz * ngb)), rblk, 0, d, hb, wzb,
-           nb, ngb, rows, h->u.as<R>(), h->v.as<R>(), h->mu.as<R>(), h->mv.as<R>(),
-           h->mx.as<R>(), h->mx2.as<R>(), h->rmu.as<R>(), h->rmv.as<R>(),
-           h->rfmzu.as<R>(), h->rfmzv.as<R>(), h->fmz.as<R>(), dtrdx, dtrdy, rot);
+  auto grid = [&](int ng) {
+    return dim3((unsigned)(((long long)ntile * nchunk * ng * d.kz + kWrWaves - 1) / kWrWaves), 1,
+                1);
+  };
+  const R *tanrot = h->tanrot.as<R>();
+  if (nb) {
+    const int ng = (nb + G - 1) / G;
+    // ux and vx go first, into one group of at least two fields, which then
+    // applies the curvature terms
+    const bool fuse = cux >= 0 && cvx == cux + 1 && nb / ng >= 2;
+    if (fuse)
+      for (int m = 0; m < 2; ++m) {
+        std::swap(hb.src[m], hb.src[cux + m]);
+        std::swap(hb.dst[m], hb.dst[cux + m]);
+        std::swap(wzb.src[m], wzb.src[cux + m]);
+      }
+    *curv = fuse;
+    MLC_EMIT(K_WAF_H, WafRRR, grid(ng), rblk, 0, d, hb, wzb, nb, ng, rows, nchunk, ntile,
+             h->u.as<R>(), h->v.as<R>(), h->mu.as<R>(), h->mv.as<R>(), h->mx.as<R>(),
+             h->mx2.as<R>(), h->rmu.as<R>(), h->rmv.as<R>(), h->rfmzu.as<R>(),
+             h->rfmzv.as<R>(), h->fmz.as<R>(), dtrdx, dtrdy, fuse ? 1 : 0, tanrot, h->rdx,
+             h->dtstepa);
+  }
   if (np) {
-    const int ngp = (np + G - 1) / G;
-    MLC_EMIT(K_WAF_H, WafRDR, dim3(gx, gy, (unsigned)(d.kz * ngp)), rblk, 0, d, hp,
-             wzp, np, ngp, rows, h->u.as<R>(), h->v.as<R>(), h->mu.as<R>(), h->mv.as<R>(),
-             h->mx.as<R>(), h->mx2.as<R>(), h->rmu.as<R>(), h->rmv.as<R>(),
-             h->rfmzu.as<R>(), h->rfmzv.as<R>(), h->fmz.as<R>(), dtrdx, dtrdy, rot);
+    const int ng = (np + G - 1) / G;
+    MLC_EMIT(K_WAF_H, WafRDR, grid(ng), rblk, 0, d, hp, wzp, np, ng, rows, nchunk, ntile,
+             h->u.as<R>(), h->v.as<R>(), h->mu.as<R>(), h->mv.as<R>(), h->mx.as<R>(),
+             h->mx2.as<R>(), h->rmu.as<R>(), h->rmv.as<R>(), h->rfmzu.as<R>(),
+             h->rfmzv.as<R>(), h->fmz.as<R>(), dtrdx, dtrdy, 0, tanrot, 0.0, 0.0);
   }
   return MLC_OK;
 }
@@ -3429,21 +3534,21 @@ static int advection(mlc_handle *h) {
                                        : waf_vertical<R, 4>(h, d, vb, nb, vp, np, dtrdz);
       if (rc) return rc;
     }
-    if (h->tune.waf_h == 0 && !d.crm) {
-      // row-streaming form (bounded domains only; a periodic domain takes
-      // the tile form, whose halo loads wrap)
-      int rc = h->tune.waf_group == 2
-                   ? waf_rows<R, 2>(h, d, hb, wzb, nb, hp, wzp, np, dtrdx, dtrdy)
-                   : waf_rows<R, 4>(h, d, hb, wzb, nb, hp, wzp, np, dtrdx, dtrdy);
+    if (h->tune.waf_h == 0) {
+      bool fused = false;
+      auto rows = [&](auto per, auto rot) {
+        return waf_rows<R, decltype(per)::value, decltype(rot)::value>(
+            h, d, hb, wzb, nb, hp, wzp, np, dtrdx, dtrdy, cux, cvx, &fused);
+      };
+      constexpr std::integral_constant<int, 0> no{};
+      constexpr std::integral_constant<int, 1> yes{};
+      const int rc = d.crm ? rows(yes, no) : rot ? rows(no, yes) : rows(no, no);
       if (rc) return rc;
+      curv = curv || fused;
     } else {
       // LDS-tile form
       int rc;
       bool fused = false;
-      // with the row-streaming form selected the curvature pass runs on its
-      // own also on a periodic domain, so that every member of a batch
-      // records the same launches
-      if (h->tune.waf_h == 0) cux = cvx = -1;
       if (d.crm)
         rc = h->tune.waf_tile == 8
                  ? waf_tile<R, 8, 1>(h, d, hb, wzb, nb, hp, wzp, np, dtrdx, dtrdy, cux, cvx, &fused)

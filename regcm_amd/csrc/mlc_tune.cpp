@@ -124,7 +124,7 @@ int autotune(mlc_handle *h, int nsteps, double *best_ms) {
     if (c <= h->g.kz) stag_vals.push_back(c);
   std::vector<Knob> knobs = {
       {&h->tune.waf_h, {0, 1}},
-      {&h->tune.waf_rows, {8, 16, 32, 64}},
+      {&h->tune.waf_rows, {4, 8, 12, 16, 32}},
       {&h->tune.waf_group, {2, 4}},
       {&h->tune.level_chunk, chunk_vals},
       {&h->tune.mom_chunk, mom_vals},

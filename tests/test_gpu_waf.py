@@ -6,12 +6,15 @@ import pytest
 
 import oracle_api as O
 from regcm_amd import synth
-from regcm_amd.moloch import MLC_VAR_WAFV_GROUP, Moloch
+from regcm_amd.moloch import (MLC_VAR_WAF_GROUP, MLC_VAR_WAF_H, MLC_VAR_WAF_ROWS,
+                              MLC_VAR_WAFV_GROUP, Moloch)
 
 pytestmark = pytest.mark.gpu
 
 
-def owned(name, a):
+def owned(g, name, a):
+    if g.crm:
+        return a
     j = a.shape[-1] if name == "u" else a.shape[-1] - 1
     i = a.shape[-2] if name == "v" else a.shape[-2] - 1
     return a[..., :i, :j]
@@ -31,7 +34,7 @@ def check(g, f, variants, label):
         m.moloch(2)
         m.synchronize()
         for n in names:
-            a, b = owned(n, ref[n]), owned(n, m.get(n))
+            a, b = owned(g, n, ref[n]), owned(g, n, m.get(n))
             assert np.array_equal(a, b), f"{label}: {n}: {np.count_nonzero(a != b)} differ"
 
 
@@ -42,6 +45,23 @@ def test_vertical_groups(kz, group, ntr):
     """6..9 fields: groups of 1 to 4 fields, full and one short."""
     g, f, _ = synth.config("small", kz=kz, jx=66, iy=11, nqx=2, ipptls=0, ntr=ntr)
     check(g, f, {MLC_VAR_WAFV_GROUP: group}, f"kz {kz} group {group} fields {6 + ntr}")
+
+
+# wave tiles: one wave holds 64 columns of a bounded domain, each further one
+# 60; a periodic domain takes 60 per wave.  Rows: chunks that end on, before
+# and past the last row
+EDGES = [("bounded", jx, iy, {}) for jx, iy in ((64, 9), (65, 10), (66, 11), (125, 12), (126, 13))] \
+    + [("rotllr", 65, 10, dict(lrotllr=1)), ("rotllr", 126, 13, dict(lrotllr=1))] \
+    + [("periodic", jx, iy, dict(crm=1)) for jx, iy in ((24, 8), (60, 9), (61, 11), (122, 13))]
+
+
+@pytest.mark.parametrize("kind,jx,iy,over", EDGES, ids=[f"{k}-{j}x{i}" for k, j, i, _ in EDGES])
+@pytest.mark.parametrize("rows,group", [(4, 2), (5, 4), (256, 4)])
+def test_row_streaming_edges(kind, jx, iy, over, rows, group):
+    g, f, _ = synth.config("crm-small" if over.get("crm") else "small", jx=jx, iy=iy, kz=5,
+                           ntr=1, **over)
+    check(g, f, {MLC_VAR_WAF_H: 0, MLC_VAR_WAF_ROWS: rows, MLC_VAR_WAF_GROUP: group},
+          f"{kind} {jx}x{iy} rows {rows} fields per wave {group}")
 
 
 def test_extreme_values():
@@ -62,7 +82,7 @@ def test_extreme_values():
         m.load(f)
         m.init_moloch()
         m.moloch(1)
-        a, b = owned("trac", ref["trac"]), owned("trac", m.get("trac"))
+        a, b = owned(g, "trac", ref["trac"]), owned(g, "trac", m.get("trac"))
         for n in range(2):
             assert np.array_equal(a[n], b[n], equal_nan=True), \
                 f"tracer {n}: {np.count_nonzero(~((a[n] == b[n]) | (np.isnan(a[n]) & np.isnan(b[n]))))}"
