@@ -216,7 +216,7 @@ int mlc_kernel_stats(mlc_handle *h, int slot, long long *launches,
 #define MLC_VAR_WAF_ROWS 1    /* row-streaming WAF: i rows per wavefront, 4..256 (by domain size) */
 #define MLC_VAR_WAF_GROUP 2   /* row-streaming WAF: fields per lane, 2 or 4 (by domain size) */
 #define MLC_VAR_LEVEL_CHUNK 3 /* divergence (and momentum, unless MLC_VAR_MOM_CHUNK is set):
-                                 levels per thread, 1..kz (8) */
+                                 levels per thread, 1..kz (by domain size) */
 #define MLC_VAR_COLUMN 4      /* column solve: 0 LDS three-phase, 1 streamed, 2 LDS with
                                  level chunks in registers (default; kz > 64 runs 0) */
 #define MLC_VAR_WAFV_GROUP 5  /* vertical WAF: fields per thread, 1, 2 or 4 (by domain
@@ -224,8 +224,8 @@ int mlc_kernel_stats(mlc_handle *h, int slot, long long *launches,
 #define MLC_VAR_XCD_MAP 6     /* single-domain launches: 1 XCD-contiguous tile order (default), 0 plain */
 #define MLC_VAR_WAF_TILE 7    /* LDS-tile WAF: output rows per tile, 4 or 8 (default 8 in FP64, 4 mixed) */
 #define MLC_VAR_WAF_HGROUP 8  /* LDS-tile WAF: fields per block, 0 = the whole batch (default) */
-#define MLC_VAR_COLUMN_J 9    /* chunked column solve: columns per block, 16, 32 (default) or
-                                 64 (up to 42 levels) */
+#define MLC_VAR_COLUMN_J 9    /* chunked column solve: columns per block, 16, 32 or 64 (up
+                                 to 42 levels; by domain size) */
 #define MLC_VAR_MIXED_MERGE 10 /* mixed form: float and double WAF batches in one launch,
                                  bit 0 vertical (default 1), bit 1 horizontal as two block
                                  ranges, bit 2 horizontal in the same blocks (one coefficient
@@ -238,7 +238,7 @@ int mlc_kernel_stats(mlc_handle *h, int slot, long long *launches,
                                  0; a non-zero mask otherwise is MLC_E_STATE.  Same bits
                                  either way. */
 #define MLC_VAR_MOM_CHUNK 12  /* momentum update: levels per thread, 1..kz, or 0 for
-                                 MLC_VAR_LEVEL_CHUNK's (default kz: whole columns) */
+                                 MLC_VAR_LEVEL_CHUNK's (by domain size) */
 #define MLC_VAR_STAGGER_CHUNK 13 /* staggering passes (winds to and from the advection
                                  grid): levels per thread, 1..kz (1) */
 #define MLC_VAR_COUNT 14

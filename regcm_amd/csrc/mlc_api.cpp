@@ -615,12 +615,37 @@ static void rows_rule(mlc_handle *const *h, int n, int *rows, int *group) {
     if (waves(r, 4) >= 12000) *rows = r;
 }
 
-void waf_shapes(mlc_handle *const *h, int n) {
-  long long waves = 0;
+// Levels per thread of the level-chunked stages (divergence, momentum) on
+// `blocks` 64 x 4 tiles: the chunk of kz / n levels that minimises
+// (levels + 1) (1 + 0.8 (blocks per CU - 1)), a block's time being its levels
+// and one start, and a further block on the same CU adding 0.8 of its own.
+// It fits the measured times to 10% between one and seven blocks per CU
+// (momentum, us: 151x127x35 at 1 / 5 / 6 / 9 / 18 chunks 21.6 / 10.6 / 12.6 /
+// 12.1 / 11.4; 500x100x60 at 1 / 4 / 5 / 8 / 10 chunks 37.0 / 34.3 / 29.3 / 33.7
+// / 30.9; 64x64x23 at 1 / 12 / 23 chunks 15.7 / 4.8 / 4.8).
+static int chunk_rule(long long blocks, int kz) {
+  int best = kz;
+  double cost = 0.0;
+  for (int n = 1; n <= kz; ++n) {
+    const int kc = (kz + n - 1) / n;
+    if ((kz + kc - 1) / kc != n) continue;
+    const double c = (kc + 1.0) * (1.0 + 0.8 * (double)((blocks * n + 255) / 256 - 1));
+    if (cost == 0.0 || c < cost) {
+      cost = c;
+      best = kc;
+    }
+  }
+  return best;
+}
+
+void launch_shapes(mlc_handle *const *h, int n) {
+  long long waves = 0, columns = 0;
   int nf = 0, rows = 0, group = 0;
   for (int m = 0; m < n; ++m) {
     waves += column_waves(h[m]->d);
     nf = h[m]->nadvf > nf ? h[m]->nadvf : nf;
+    columns += (long long)((h[m]->d.jc2 - h[m]->d.jc1 + 32) / 32) *
+               (h[m]->d.ic2 - h[m]->d.ic1 + 1);
   }
   const int wafv = wafv_rule(waves, nf);
   rows_rule(h, n, &rows, &group);
@@ -628,6 +653,16 @@ void waf_shapes(mlc_handle *const *h, int n) {
     h[m]->tune.wafv_group = wafv;
     h[m]->tune.waf_rows = rows;
     h[m]->tune.waf_group = group;
+    // a domain that fills the chip with one level chunk keeps 8 levels in the
+    // divergence, and in FP64 whole columns in the momentum update (31.7 us
+    // against 36.9 in four chunks at 256x256x41, where both stream from HBM)
+    const int kz = h[m]->g.kz, kc = chunk_rule(waves / 4, kz);
+    const bool full = waves >= 1024;
+    h[m]->tune.level_chunk = full ? (kz < 8 ? kz : 8) : kc;
+    h[m]->tune.mom_chunk = full && !h[m]->mixed ? kz : kc;
+    // 16 columns per block while 32 leave CUs without one: 64x64x23 11.4 ->
+    // 9.0 us, 100x50x30 mixed 11.8 -> 10.7; 151x127x35 loses, 20.7 -> 22.3
+    h[m]->tune.column_j = columns <= 256 ? 16 : 32;
   }
 }
 
@@ -659,9 +694,6 @@ int create_handle(const mlc_grid_desc *g, hipStream_t shared, mlc_handle **out) 
   // 4 for the mixed form, whose float tiles leave room for more blocks: what
   // the autotuner chose at 256 x 256 x 41, 512 x 512 x 41 and 100 x 50 x 30
   h->tune.waf_tile = h->mixed ? 4 : 8;
-  // the momentum update streams whole columns (fastest at 256x256x41 in
-  // FP64, 20.3 against 21.8 us in the mixed form)
-  h->tune.mom_chunk = g->kz;
   h->d = mlc::make_dims(g->jx, g->iy, g->kz, g->crm);
   // advected slots in the order of advection (Main/mod_moloch.F90:786-808):
   // tetav, pai, ux, vx, wx, qv, qx(iqfrst:nqx) with ipptls > 0, tkex, trac
@@ -677,7 +709,7 @@ int create_handle(const mlc_grid_desc *g, hipStream_t shared, mlc_handle **out) 
     h->s_tr0 = h->nslots;
     for (int n = 0; n < g->ntr; ++n) h->adv_list[h->nadvf++] = h->nslots++;
   }
-  waf_shapes(&h, 1);
+  launch_shapes(&h, 1);
   h->h_mx.assign((size_t)h->d.plane, 0.0);
   h->h_mu.assign((size_t)h->d.plane, 0.0);
   h->h_mv.assign((size_t)h->d.plane, 0.0);

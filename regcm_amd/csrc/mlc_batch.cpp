@@ -262,7 +262,7 @@ int mlc_batch_create(const mlc_grid_desc *descs, int n, mlc_batch **out) {
     b->npoints += mlc_npoints(h);
   }
   // the members' launches are merged: one choice, by their common grid
-  waf_shapes(b->all.data(), n);
+  launch_shapes(b->all.data(), n);
   *out = b;
   return MLC_OK;
 }

@@ -297,17 +297,17 @@ struct mlc_handle {
   // launch-shape choices (autotuned per domain shape)
   struct Tune {
     int waf_h = 0;               // horizontal WAF: 0 row-streaming, 1 LDS tile
-    int waf_rows = 16;           // row-streaming WAF: i rows per wavefront (waf_shapes)
-    int waf_group = 4;           // row-streaming WAF: fields per lane (2 or 4; waf_shapes)
-    int level_chunk = 8;         // divergence/momentum: levels per thread
+    int waf_rows = 16;           // row-streaming WAF: i rows per wavefront (launch_shapes)
+    int waf_group = 4;           // row-streaming WAF: fields per lane (2 or 4; launch_shapes)
+    int level_chunk = 8;         // divergence/momentum: levels per thread (launch_shapes)
     int mom_chunk = 0;           // momentum, if not 0: levels per thread
     int stag_chunk = 1;          // staggering passes: levels per thread
     int column = 2;              // column solve: 0 LDS three-phase, 1 streamed, 2 chunked
-    int wafv_group = 4;          // vertical WAF: fields per thread (1, 2 or 4; waf_shapes)
+    int wafv_group = 4;          // vertical WAF: fields per thread (1, 2 or 4; launch_shapes)
     int xcd_map = 1;             // XCD-contiguous tile order of single-domain launches
     int waf_tile = 4;            // LDS-tile WAF: output rows per tile (4 or 8; FP64 starts at 8)
     int waf_hgroup = 0;          // LDS-tile WAF: fields per block (0 = the whole batch)
-    int column_j = 32;           // chunked column solve: columns per block (16 or 32)
+    int column_j = 32;           // chunked column solve: columns per block (launch_shapes)
     int mixed_merge = 1;         // mixed form: float and double WAF batches in one launch
                                  // (bit 0 vertical, bit 1 horizontal)
     int terrain = 0;             // stages forming the terrain metrics from the orography
@@ -325,9 +325,9 @@ struct mlc_handle {
 
 namespace mlc {
 
-// Sets the WAF launch shapes of handles whose stages run in common launches
-// (one handle, or a batch's members) from their sizes.
-void waf_shapes(mlc_handle *const *h, int n);
+// Sets the launch shapes of handles whose stages run in common launches (one
+// handle, or a batch's members) from their sizes.
+void launch_shapes(mlc_handle *const *h, int n);
 
 // Error reporting (thread-local message).
 int fail(int code, const std::string &msg);
