@@ -138,6 +138,23 @@ struct BdyWt {
   }
 };
 
+// 1 / x, correctly rounded, for a normal x whose reciprocal is normal.  The
+// hardware's estimate (2^-24) takes one third-order step, after which it is
+// within an ulp, and its exact remainder (Markstein's correction).  The
+// compiler's own division also scales both operands against overflow and
+// underflow: 11 dependent instructions against 6.  Zero, infinite and NaN
+// operands need v_div_fixup (recip).
+__device__ __forceinline__ double recip_normal(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  double e = __builtin_fma(-x, y, 1.0);
+  e = __builtin_fma(e, e, e);
+  y = __builtin_fma(y, e, y);
+  return __builtin_fma(__builtin_fma(-x, y, 1.0), y, y);
+}
+__device__ __forceinline__ double recip(double x) {
+  return __builtin_amdgcn_div_fixup(recip_normal(x), x, 1.0);
+}
+
 // The terrain-following metrics of compute_moloch_static
 // (Main/mod_params.F90:3356-3385) formed from the surface geopotential:
 //   fmz(j,i,k)   = 1/(gzitap(zitah(k))*orog + bzitap(zitah(k))),  orog = ht*regrav
@@ -145,7 +162,7 @@ struct BdyWt {
 //   rfmzu(j,i,k) = 1/md_fmz(zitah(k), htu(j,i)),  rfmzv on htv
 // (md_fmz / md_fmz_h, Share/mod_zita.F90:135-141, 165-170), with the same
 // operations in the same order as the reference, so each value is the one
-// the caller computed.  gzitap and bzitap are per-level tables; ht, htu, htv
+// the caller computed.  The divisions are recip_normal, in the check too.  gzitap and bzitap are per-level tables; ht, htu, htv
 // are 2-D.  `on` is set only after mlc_init has compared the formula with
 // every uploaded metric bit for bit, and then per stage; otherwise the
 // kernels stream the uploaded 3-D arrays.
@@ -153,22 +170,18 @@ struct ZMet {
   const double *ga, *ba;   // gzitap, bzitap: zitah(1..kz) then zita(1..kz+1)
   const double *hc, *hu, *hv;   // ht, htu, htv (m2/s2), [iy][pj]
   int kz, on;
-  __host__ __device__ double den(const double *h, long long c2, int t) const {
+  __device__ double den(const double *h, long long c2, int t) const {
     return ga[t] * (h[c2] * kRegrav) + ba[t];
   }
-  __host__ __device__ double fmz(long long c2, int k) const { return 1.0 / den(hc, c2, k - 1); }
-  __host__ __device__ double fmzf(long long c2, int k) const {
-    return 1.0 / den(hc, c2, kz + k - 1);
+  __device__ double fmz(long long c2, int k) const { return recip_normal(den(hc, c2, k - 1)); }
+  __device__ double fmzf(long long c2, int k) const {
+    return recip_normal(den(hc, c2, kz + k - 1));
   }
-  __host__ __device__ double rfmzu(long long c2, int k) const {
-    return 1.0 / (1.0 / den(hu, c2, k - 1));
-  }
-  __host__ __device__ double rfmzv(long long c2, int k) const {
-    return 1.0 / (1.0 / den(hv, c2, k - 1));
-  }
+  __device__ double rfmzu(long long c2, int k) const { return rfm(hu, c2, k); }
+  __device__ double rfmzv(long long c2, int k) const { return rfm(hv, c2, k); }
   // rfmzu (h = hu) or rfmzv (h = hv)
-  __host__ __device__ double rfm(const double *h, long long c2, int k) const {
-    return 1.0 / (1.0 / den(h, c2, k - 1));
+  __device__ double rfm(const double *h, long long c2, int k) const {
+    return recip_normal(recip_normal(den(h, c2, k - 1)));
   }
 };
 

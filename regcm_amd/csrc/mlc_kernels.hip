@@ -432,7 +432,7 @@ __device__ __forceinline__ void SoundColumn<R>::run(const SoundColumn &args_, in
     double wk_up = 0.0, w_up = wtop;                               // wwkw(kz+1) = 0
     for (int k = kz; k >= 2; --k) {
       const double zu = s_zu[k * kColJ + tx], zd = s_zd[k * kColJ + tx];
-      const double zrapp = 1.0 / (1.0 + zd + zu - zd * wk_up);
+      const double zrapp = recip(1.0 + zd + zu - zd * wk_up);
       const double wt = zrapp * (s_rh[k * kColJ + tx] + zd * w_up);
       const double wkk = zrapp * zu;
       s_rh[k * kColJ + tx] = wt;
@@ -461,20 +461,31 @@ __device__ __forceinline__ void SoundColumn<R>::run(const SoundColumn &args_, in
 }
 
 // The same column stage with each thread owning a contiguous chunk of at
-// most CC levels of its column: the filtered divergence z2 of its levels
-// (and of the level above its chunk) stays in registers, so LDS holds only
-// the three tridiagonal arrays (zu, zd, rhs) and the stage needs two
-// barriers.  CJ columns per block (along j), CK threads per column, at
-// most CC levels per thread; requires kz <= CK * CC, and runs with the
-// smallest CC that holds the column (6 or 3 for kz <= 48, else 8) so that
-// no thread carries unused levels.  Same operations as SoundColumn.
+// most CC levels of its column, whose z2, pai, metrics and tetavf stay in
+// registers, so LDS holds only the three tridiagonal arrays (zu, zd, rhs) and
+// level tables.  CJ columns per block (along j), CK threads per column;
+// requires kz <= CK * CC, and runs with the smallest CC that holds the column
+// (6 or 3 for kz <= 48, else 8) so that no thread carries unused levels.  Same
+// operations as SoundColumn.
+//
+// Large domains are bound by memory: every array is read once, also across
+// the chunks (a thread passes its last level's values on through LDS), no
+// store stands before a load, and a few levels' loads are always in flight
+// within the registers of four waves per SIMD.  Small domains are bound by the
+// chain of kz divisions, which reads LDS a level ahead and takes the short
+// reciprocal.  Measured per call, before (a chunk's neighbour level formed
+// twice, one level's inputs in flight, tetavf stored as it is formed) and
+// after: 256x256x41 FP64 49.2 -> 45.2 us (4.3 TB/s over its 9 arrays), mixed
+// 46.8 -> 42.2, 500x100x60 64.6 -> 57.4, 8 x 128x128x30 99.5 -> 82.9,
+// 151x127x35 21.1 -> 19.2, 64x64x23 9.4 -> 9.1.
 constexpr int kColC = 8;
 
 // LDS of a chunked column block of cj columns: the three tridiagonal arrays
-// of levels 2..kz and the interleaved gzitap / bzitap tables (2 kz + 1
-// levels each) of the formed terrain metrics
+// of levels 2..kz, the level tables xknu and ffilt, and the interleaved
+// gzitap / bzitap tables (2 kz + 1 levels each) of the formed terrain metrics
 inline size_t col_chunk_lds(int kz, int cj) {
-  return (3 * (size_t)(kz - 1) * cj + 2 * (size_t)(2 * kz + 1)) * sizeof(double);
+  return (3 * (size_t)(kz - 1) * cj + 2 * (size_t)kz + 2 * (size_t)(2 * kz + 1)) *
+         sizeof(double);
 }
 
 template <typename R, int CJ, int CK, int CC = kColC>
@@ -510,11 +521,12 @@ __device__ __forceinline__ void SoundColumnChunk<R, CJ, CK, CC>::run(
   const int divfilter = args_.divfilter, first = args_.first;
   const ZMet zm = args_.zm;
   const int kz = d.kz;
-  // levels 2..kz of the tridiagonal arrays, level k at row k - 2; then,
-  // with the formed metrics, gzitap and bzitap of every level, interleaved
+  // levels 2..kz of the tridiagonal arrays, level k at row k - 2; then the
+  // level tables and, with the formed metrics, gzitap and bzitap of every
+  // level, interleaved
   const int L = (kz - 1) * CJ;
   double *s_zu = smem, *s_zd = smem + L, *s_rh = smem + 2 * L;
-  double *s_gb = smem + 3 * L;
+  double *s_xk = smem + 3 * L, *s_ff = s_xk + kz, *s_gb = s_ff + kz;
   const int tx = threadIdx.x, ty = threadIdx.y;
   const int j = d.jc1 + bx * CJ + tx;
   const int i = d.ic1 + by;
@@ -527,137 +539,236 @@ __device__ __forceinline__ void SoundColumnChunk<R, CJ, CK, CC>::run(
   const int kc = (kz + CK - 1) / CK;
   const int ka = 1 + ty * kc;                       // first level of the chunk
   const int kb = ka + kc - 1 < kz ? ka + kc - 1 : kz;
-  // w(1) and w(kz+1) are not written by this stage; their loads are issued
-  // first so that their latency overlaps phase 1.  Lanes past the domain
-  // (!ok) load from the valid column c1 and store nothing.
-  const double w1 = w[c1];                                         // w(1)
-  const double wtop = w[c1 + (long long)kz * P];                   // w(kz+1)
-  // The formed metrics' per-level tables are read from LDS and the
-  // orography term ht(j,i)*regrav is loaded once: read from global memory
-  // at every level, each division waited for its own table loads (and ht
-  // was loaded again after every tetavf store, which could alias it).
-  // the boundary-weight column (its index load, on which every weight's
-  // address depends, goes out before the tables' barrier)
+  // The order of the loads is the order of the waits: the boundary-weight
+  // column's index, on which the weights' addresses depend, and the level
+  // tables first, then every array of the chunk.  Nothing is stored before
+  // the last load (a load behind a store waits for the store), tetavf too
+  // waits in registers for the end.  Loads read a level clamped into the
+  // column; lanes past the domain (!ok) read the valid column c1 and store
+  // nothing.
+  // w(1) and w(kz+1) are not written by this stage
+  const double w1 = w[c1], wtop = w[c1 + (long long)kz * P];
+  // z2r[m], pr[m], fr[m], tvf[m] = z2, pai, fmz, tetavf of level ka + m: they
+  // stay in registers for the Exner update
+  double z2r[CC], pr[CC], fr[CC], tvf[CC];
+  // phase 1 with the metrics formed from the orography (ZC) or streamed, with
+  // the divergence filter (DF) or without
+  auto phase1 = [&](auto zc_, auto df_) __attribute__((always_inline)) {
+  constexpr bool zc = decltype(zc_)::value, df = decltype(df_)::value;
   const R *__restrict__ bcol = bdw.col(c2);
-  double hreg = 0.0;
-  if (zm.on) {
-    hreg = zm.hc[c2] * kRegrav;
-    for (int t = ty * CJ + tx; t < 2 * kz + 1; t += CJ * CK) {
+  const int t0 = ty * CJ + tx;
+  const double hreg = zc ? zm.hc[c2] * kRegrav : 0.0;
+  const double txk = t0 < kz ? xknu[t0] : 0.0, tff = t0 < kz ? ffilt[t0] : 0.0;
+  const int tg = t0 <= 2 * kz ? t0 : 2 * kz;
+  const double tga = zc ? zm.ga[tg] : 0.0, tba = zc ? zm.ba[tg] : 0.0;
+  // byte offsets of the column's points in an array of T (the launcher keeps
+  // arrays below 4 GiB): one register per level, the bases stay uniform
+  const unsigned u1 = (unsigned)c1, uP = (unsigned)P;
+  auto ld = [](auto *p, unsigned o) {
+    return *(decltype(p))((const char *)p + o * (unsigned)sizeof(*p));
+  };
+  auto at = [&](int m, int top) {
+    const int k = ka + m;
+    return u1 + (unsigned)((k > top ? top : k) - 1) * uP;
+  };
+  const unsigned uw = (unsigned)ow, ue = (unsigned)oe, us = (unsigned)os, un = (unsigned)on;
+  R zr[CC][5], sr[CC + 1], bw[CC];
+  double ff[CC], tv[CC + 1], wr[CC], tf[CC];
+  auto load = [&](int m) __attribute__((always_inline)) {
+    const unsigned c = at(m, kz);
+    zr[m][0] = ld(zdiv2, c);
+    if constexpr (df) {
+      zr[m][1] = ld(zdiv2, c + uw);
+      zr[m][2] = ld(zdiv2, c + ue);
+      zr[m][3] = ld(zdiv2, c + us);
+      zr[m][4] = ld(zdiv2, c + un);
+    }
+    sr[m + 1] = ld(s, at(m + 1, kz + 1));          // s has a level kz + 1
+    pr[m] = ld(pai, c);
+    bw[m] = bcol[(ka + m < kz ? ka + m : kz) - 1];
+    if constexpr (!zc) fr[m] = ld(fmz, c);
+  };
+  // the coefficients' own inputs; tv[m] = tetav(ka - 1 + m).  The first
+  // sub-step forms tetavf from tetav and reads nothing else.
+  const double *__restrict__ tfp = first ? tetav : tetavf;
+  auto fetch = [&](int m) __attribute__((always_inline)) {
+    const unsigned c = at(m, kz);
+    tv[m + 1] = ld(tetav, c);
+    wr[m] = ld(w, c);
+    tf[m] = ld(tfp, c);
+    if constexpr (!zc) ff[m] = ld(fmzf, c);
+  };
+  // NB levels of the first kind are in flight together; as each is used the
+  // next goes out, then the second kind (with few registers per level
+  // everything goes out before the first wait).
+  constexpr bool kAll = CC <= 3;
+  constexpr int NB = CC <= 4 ? CC : (sizeof(R) == 4 ? 4 : 2);
+  sr[0] = ld(s, at(0, kz));
+#pragma unroll
+  for (int m = 0; m < NB; ++m) load(m);
+  if constexpr (kAll) {
+    tv[0] = ld(tetav, ty ? at(-1, kz) : u1);
+#pragma unroll
+    for (int m = 0; m < CC; ++m) fetch(m);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (t0 < kz) {
+    s_xk[t0] = txk;
+    s_ff[t0] = tff;
+  }
+  if (zc && t0 <= 2 * kz) {
+    s_gb[2 * t0] = tga;
+    s_gb[2 * t0 + 1] = tba;
+  }
+  if constexpr (zc) {
+    for (int t = t0 + CJ * CK; t <= 2 * kz; t += CJ * CK) {
       s_gb[2 * t] = zm.ga[t];
       s_gb[2 * t + 1] = zm.ba[t];
     }
-    __syncthreads();
   }
+  __syncthreads();
   // ZMet::fmz(c2, k) = 1 / den(t = k - 1), fmzf(c2, k) = 1 / den(t = kz + k - 1)
   auto zden = [&](int t) { return s_gb[2 * t] * hreg + s_gb[2 * t + 1]; };
-  // z2r[m], pr[m], fr[m] = z2, pai, fmz of level ka - 1 + m, m = 0 .. kc;
-  // pai and fmz of the chunk stay in registers for the Exner update.
-  // Phase 1 is branch-free up to its stores: every load reads a level
-  // clamped into the column and the unused values are masked, so the loads
-  // of all levels can be in flight together.
-  double z2r[CC + 1], pr[CC + 1], fr[CC + 1];
-  // phase 1 with the metrics formed from the orography (ZC) or streamed
-  auto phase1 = [&](auto zc) __attribute__((always_inline)) {
-    constexpr bool ZC = decltype(zc)::value;
-    auto z2_levels = [&](auto df) {
-#pragma unroll
-      for (int m = 0; m <= CC; ++m) {
-        const int k = ka - 1 + m;
-        const bool in = m <= kb - ka + 1 && k >= 1;
-        const int kk = k < 1 ? 1 : (k > kz ? kz : k);
-        const long long c = c1 + (long long)(kk - 1) * P;
-        const double fzk = ZC ? 1.0 / zden(kk - 1) : fmz[c], pk = pai[c];
-        double z = zdiv2[c];
-        if (decltype(df)::value) {
-          const double lap = ((double)zdiv2[c + ow] + (double)zdiv2[c + oe] +
-                              (double)zdiv2[c + os] + (double)zdiv2[c + on] - 4.0 * z);
-          z = z + xknu[kk - 1] * lap;
-        }
-        z = z + (double)bcol[kk - 1] * dtrdz * fzk * ((double)s[c] - (double)s[c + P]);
-        fr[m] = in ? fzk : 0.0;
-        pr[m] = in ? pk : 0.0;
-        z2r[m] = in ? z : 0.0;
-      }
-    };
-    if (divfilter)
-      z2_levels(std::true_type{});
-    else
-      z2_levels(std::false_type{});
-    // the tridiagonal coefficients of levels ka .. kb (>= 2); the inputs of
-    // the next level are loaded before this level's stores
-    auto lev = [&](int m) {
-      const int k = ka - 1 + m;
-      return k < 2 ? 2 : (k > kz ? kz : k);
-    };
-    double q_tv, q_tm, q_tf, q_w, q_fz, q_ff;
-    auto fetch = [&](int m) {
-      const long long c = c1 + (long long)(lev(m) - 1) * P;
-      q_tv = tetav[c];
-      q_tm = tetav[c - P];
-      q_tf = tetavf[c];
-      q_w = w[c];
-      q_fz = ZC ? 1.0 / zden(kz + lev(m) - 1) : fmzf[c];
-      q_ff = ffilt[lev(m) - 1];
-    };
-    fetch(1);
-#pragma unroll
-    for (int m = 1; m <= CC; ++m) {
-      const double tvk = q_tv, tvkm1 = q_tm, tvf0 = q_tf, wk = q_w, fzf = q_fz, ffk = q_ff;
-      if (m < CC) fetch(m + 1);
-      const int k = ka - 1 + m;
-      double tvf = first ? 0.5 * (tvkm1 + tvk) : tvf0;
-      tvf = tvf - wk * fzf * dtrdz * (tvkm1 - tvk);
-      const double zrom1w = kCpd * tvf * fzf;
-      const double pk = pr[m], pkm1 = pr[m - 1];
-      const double zkm1 = z2r[m - 1], zk = z2r[m];
-      double zwexpl = wk - zrom1w * dtrdz * (pkm1 - pk) - kEgrav * dts;
-      zwexpl = zwexpl + kRdrcv * zrom1w * dtrdz * (pkm1 * zkm1 - pk * zk);
-      const double zu = zcs2 * fr[m - 1] * zrom1w * pkm1 + ffk;
-      const double zd = zcs2 * fr[m] * zrom1w * pk + ffk;
-      if (ok && k <= kb && k >= 2) {
-        tetavf[c1 + (long long)(k - 1) * P] = tvf;
-        s_zu[(k - 2) * CJ + tx] = zu;
-        s_zd[(k - 2) * CJ + tx] = zd;
-        s_rh[(k - 2) * CJ + tx] = zwexpl;
-      }
+  // The next thread of the column needs z2, pai and fmz of level kb: they
+  // pass through its own first rows in LDS.
+  auto level = [&](int m) __attribute__((always_inline)) {
+    // a level at a time: the scheduler would otherwise gather every level's
+    // table reads above the first use, at 10 registers each
+    __builtin_amdgcn_sched_barrier(0);
+    const int kk = ka + m < kz ? ka + m : kz;
+    if constexpr (zc) fr[m] = recip_normal(zden(kk - 1));
+    double z = zr[m][0];
+    if constexpr (df) {
+      const double lap = ((double)zr[m][1] + (double)zr[m][2] + (double)zr[m][3] +
+                          (double)zr[m][4] - 4.0 * z);
+      z = z + s_xk[kk - 1] * lap;
+    }
+    z2r[m] = z + (double)bw[m] * dtrdz * fr[m] * ((double)sr[m] - (double)sr[m + 1]);
+    if (m == kc - 1 && ka + m < kz) {
+      const int o = (ka + m - 1) * CJ + tx;        // row of level kb + 1
+      s_zu[o] = z2r[m];
+      s_zd[o] = pr[m];
+      s_rh[o] = fr[m];
     }
   };
-  if (ka <= kz) {
-    if (zm.on)
-      phase1(std::true_type{});
+#pragma unroll
+  for (int m = 0; m < CC; ++m) {
+    level(m);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!kAll) {
+      if (m + NB < CC) {
+        load(m + NB);
+      } else {
+        if (m + NB == CC) tv[0] = ld(tetav, ty ? at(-1, kz) : u1);
+        // CC coefficient loads over the last NB levels
+        const int q = m + NB - CC;
+#pragma unroll
+        for (int f = q * CC / NB; f < (q + 1) * CC / NB; ++f) fetch(f);
+      }
+    }
+  }
+  __syncthreads();
+  double zkm1 = 0.0, pkm1 = 0.0, fkm1 = 0.0;     // level ka - 1
+  if (ty) {
+    const int o = (ka < kz ? ka - 2 : kz - 2) * CJ + tx;
+    zkm1 = s_zu[o];
+    pkm1 = s_zd[o];
+    fkm1 = s_rh[o];
+  }
+#pragma unroll
+  for (int m = 0; m < CC; ++m) {
+    __builtin_amdgcn_sched_barrier(0);
+    const int k = ka + m;
+    const double tvk = tv[m + 1], tvkm1 = tv[m], wk = wr[m];
+    const int kf = k < kz ? k : kz;
+    const double fzf = zc ? recip_normal(zden(kz + kf - 1)) : ff[m];
+    const double ffk = s_ff[kf - 1];
+    double t = first ? 0.5 * (tvkm1 + tvk) : tf[m];
+    t = t - wk * fzf * dtrdz * (tvkm1 - tvk);
+    tvf[m] = t;
+    const double zrom1w = kCpd * t * fzf;
+    const double pk = pr[m], zk = z2r[m], fk = fr[m];
+    double zwexpl = wk - zrom1w * dtrdz * (pkm1 - pk) - kEgrav * dts;
+    zwexpl = zwexpl + kRdrcv * zrom1w * dtrdz * (pkm1 * zkm1 - pk * zk);
+    const double zu = zcs2 * fkm1 * zrom1w * pkm1 + ffk;
+    const double zd = zcs2 * fk * zrom1w * pk + ffk;
+    if (k <= kb && k >= 2) {
+      s_zu[(k - 2) * CJ + tx] = zu;
+      s_zd[(k - 2) * CJ + tx] = zd;
+      s_rh[(k - 2) * CJ + tx] = zwexpl;
+    }
+    zkm1 = zk;
+    pkm1 = pk;
+    fkm1 = fk;
+  }
+  };
+  if (zm.on) {
+    if (divfilter)
+      phase1(std::true_type{}, std::true_type{});
     else
-      phase1(std::false_type{});
+      phase1(std::true_type{}, std::false_type{});
+  } else {
+    if (divfilter)
+      phase1(std::false_type{}, std::true_type{});
+    else
+      phase1(std::false_type{}, std::false_type{});
   }
   __syncthreads();
   if (ok && ty == 0) {
+    // The two recurrences, one dependent chain per column.  Every level's
+    // coefficients are read from LDS ahead of the chain: a level in the
+    // elimination, whose step is a division long, four in the substitution.
     double wk_up = 0.0, w_up = wtop;                               // wwkw(kz+1) = 0
-    for (int k = kz; k >= 2; --k) {
-      const double zu = s_zu[(k - 2) * CJ + tx], zd = s_zd[(k - 2) * CJ + tx];
-      const double zrapp = 1.0 / (1.0 + zd + zu - zd * wk_up);
-      const double wt = zrapp * (s_rh[(k - 2) * CJ + tx] + zd * w_up);
-      const double wkk = zrapp * zu;
-      s_rh[(k - 2) * CJ + tx] = wt;
-      s_zu[(k - 2) * CJ + tx] = wkk;
-      w_up = wt;
-      wk_up = wkk;
+    double *pu = s_zu + tx, *pd = s_zd + tx, *pw = s_rh + tx;
+    double zu = pu[(kz - 2) * CJ], zd = pd[(kz - 2) * CJ], rh = pw[(kz - 2) * CJ];
+    for (int r = kz - 2; r >= 0; --r) {
+      const int q = (r ? r - 1 : 0) * CJ;
+      const double nu = pu[q], nd = pd[q], nr = pw[q];
+      const double zrapp = recip(1.0 + zd + zu - zd * wk_up);
+      w_up = zrapp * (rh + zd * w_up);
+      wk_up = zrapp * zu;
+      pw[r * CJ] = w_up;
+      pu[r * CJ] = wk_up;
+      zu = nu;
+      zd = nd;
+      rh = nr;
     }
-    double below = w1;
-    for (int k = 2; k <= kz; ++k) {
-      const double wf = s_rh[(k - 2) * CJ + tx] + s_zu[(k - 2) * CJ + tx] * below;
-      s_rh[(k - 2) * CJ + tx] = wf;
-      below = wf;
+    double below = w1, wt[4], wk[4];
+    const int last = kz - 2;
+    auto read = [&](int r, double (&t)[4], double (&c)[4]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const int q = (r + m < last ? r + m : last) * CJ;
+        t[m] = pw[q];
+        c[m] = pu[q];
+      }
+    };
+    read(0, wt, wk);
+    for (int r = 0; r <= last; r += 4) {
+      double nt[4], nc[4];
+      read(r + 4, nt, nc);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        below = wt[m] + wk[m] * below;
+        if (r + m <= last) pw[(r + m) * CJ] = below;
+        wt[m] = nt[m];
+        wk[m] = nc[m];
+      }
     }
   }
   __syncthreads();
-  if (ok && ka <= kz) {
+  if (ok) {
 #pragma unroll
-    for (int m = 1; m <= CC; ++m) {
-      const int k = ka - 1 + m;
+    for (int m = 0; m < CC; ++m) {
+      const int k = ka + m;
       if (k <= kb) {
         const long long c = c1 + (long long)(k - 1) * P;
         const double wk = (k == 1) ? w1 : s_rh[(k - 2) * CJ + tx];
         const double wkp1 = (k == kz) ? wtop : s_rh[(k - 1) * CJ + tx];
-        if (k >= 2) w[c] = wk;
+        if (k >= 2) {
+          w[c] = wk;
+          tetavf[c] = tvf[m];
+        }
         pai[c] = pr[m] * (1.0 - kRdrcv * (z2r[m] + (dtrdz * fr[m] * (wk - wkp1))));
       }
     }
@@ -743,7 +854,7 @@ __device__ __forceinline__ void SoundColumnStream<R>::run(const SoundColumnStrea
     zwexpl = zwexpl + kRdrcv * zrom1w * dtrdz * (pai_km1 * z_km1 - pai_k * z_k);
     const double zu = zcs2 * fmz_km1 * zrom1w * pai_km1 + ffilt[k - 1];
     const double zd = zcs2 * fmz_k * zrom1w * pai_k + ffilt[k - 1];
-    const double zrapp = 1.0 / (1.0 + zd + zu - zd * wk_up);
+    const double zrapp = recip(1.0 + zd + zu - zd * wk_up);
     const double wt = zrapp * (zwexpl + zd * w_up);
     const double wkk = zrapp * zu;
     wtb[c] = wt;
@@ -1004,7 +1115,7 @@ __device__ __forceinline__ void StaggerIn<R>::run(const StaggerIn &args_, int bx
     const R w0 = R(w0d), w1 = R(w1d), w2 = R(w2d), wm = R(wmd);
     wx[c] = (k == 1 || k == kz) ? h * (w1 + w0) : a9 * (w1 + w0) - a1 * (w2 + wm);
     if (inner) {
-      const R fz = zm.on ? R(1.0 / (zg * (zh * kRegrav) + zb)) : fzs;
+      const R fz = zm.on ? R(recip_normal(zg * (zh * kRegrav) + zb)) : fzs;
       s[c] = k >= 2 ? (w0 + sc) * fz : R(0);
       if (k == kz) s[c + P] = R(0);
     }
@@ -1378,11 +1489,12 @@ __device__ __forceinline__ void waf_h_body(const WafHorizontal<T, S, TR, PER> &a
   };
   const double zga = zm.on ? zm.ga[k - 1] : 0.0, zba = zm.on ? zm.ba[k - 1] : 0.0;
   auto f_fz = [&](M raw) -> S {
-    if constexpr (kRaw) return zm.on ? S(1.0 / (zga * (raw * kRegrav) + zba)) : S(raw);
+    if constexpr (kRaw) return zm.on ? S(recip_normal(zga * (raw * kRegrav) + zba)) : S(raw);
     else return raw;
   };
   auto f_rf = [&](M raw) -> S {
-    if constexpr (kRaw) return zm.on ? S(1.0 / (1.0 / (zga * (raw * kRegrav) + zba))) : S(raw);
+    if constexpr (kRaw)
+      return zm.on ? S(recip_normal(recip_normal(zga * (raw * kRegrav) + zba))) : S(raw);
     else return raw;
   };
   S y_zamu[kPyM], y_hv[kPyM], y_is[kPyM];
@@ -3162,6 +3274,11 @@ template <typename R> struct XcdOrder<Slice<R>> { static constexpr bool value = 
 // it spills 22 to scratch and still runs a 256 x 256 x 41 domain in one
 // round instead of 1.33 (170 -> 126 us).  Tail<float> reaches 6 without
 // spilling.
+// The column solve's loads and its chunk of every array, held for the update,
+// fit four waves per SIMD up to eight levels per thread.
+template <typename R, int CJ, int CK, int CC> struct MinWaves<SoundColumnChunk<R, CJ, CK, CC>> {
+  static constexpr int value = CC <= 6 ? 4 : CC <= 8 ? 3 : 2;
+};
 template <> struct MinWaves<Slice<double>> { static constexpr int value = 4; };
 template <> struct MinWaves<Tail<float>> { static constexpr int value = 6; };
 
@@ -3251,6 +3368,9 @@ static int sound_substep(mlc_handle *h, bool first) {
     column_j = 16;
   }
   if (column == 2 && d.kz > 16 * kColC) column = 1;
+  // its byte offsets are 32 bits wide
+  if (column == 2 && (unsigned long long)d.plane * (d.kz + 1) * sizeof(double) >= 1ull << 32)
+    column = 1;
   if (column == 2 && column_j == 64) {
     const dim3 cgrid = grid_columns(d, 64);
     const size_t lds = col_chunk_lds(d.kz, 64);
