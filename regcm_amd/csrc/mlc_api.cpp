@@ -954,13 +954,18 @@ int mlc_init(mlc_handle *h) {
 int mlc_reset_tendencies(mlc_handle *h) {
   if (!h) return fail(MLC_E_ARG, "null handle");
   const long long n3 = h->d.plane * h->d.kz;
-  int rc;
-  if ((rc = launch_fill(h, h->tten, n3, 0.0))) return rc;
-  if ((rc = launch_fill(h, h->uten, n3, 0.0))) return rc;
-  if ((rc = launch_fill(h, h->vten, n3, 0.0))) return rc;
-  if ((rc = launch_fill(h, h->qxten, n3 * h->g.nqx, 0.0))) return rc;
-  if (h->s_tkex >= 0 && (rc = launch_fill(h, h->tketen, n3 + h->d.plane, 0.0))) return rc;
-  if (h->s_tr0 >= 0 && (rc = launch_fill(h, h->chiten, n3 * h->g.ntr, 0.0))) return rc;
+  const Buf *b[6] = {&h->tten, &h->uten, &h->vten, &h->qxten};
+  long long n[6] = {n3, n3, n3, n3 * h->g.nqx};
+  int count = 4;
+  if (h->s_tkex >= 0) {
+    b[count] = &h->tketen;
+    n[count++] = n3 + h->d.plane;
+  }
+  if (h->s_tr0 >= 0) {
+    b[count] = &h->chiten;
+    n[count++] = n3 * h->g.ntr;
+  }
+  if (const int rc = launch_zero(h, b, n, count)) return rc;
   h->tend_dirty = false;
   return MLC_OK;
 }
@@ -1097,9 +1102,7 @@ int mlc_step_lbc(mlc_handle *h, int nsteps, const double *x1) {
   for (int n = 0; n < nsteps; ++n) {
     if (h->tend_dirty && (rc = mlc_reset_tendencies(h))) return rc;
     if ((rc = mlc_dynamical_core(h))) return rc;
-    if ((rc = launch_boundary(h, x1[n]))) return rc;
-    if ((rc = launch_diagnostics(h))) return rc;
-    if ((rc = launch_status_update(h, h->g.dtsec))) return rc;
+    if ((rc = launch_boundary_step(h, x1[n]))) return rc;
   }
   return MLC_OK;
 }

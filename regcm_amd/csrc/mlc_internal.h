@@ -396,8 +396,12 @@ int launch_status_update(mlc_handle *h, double dtinc);
 // whose tendencies are zero (physics off)
 int launch_step_tail(mlc_handle *h);
 int launch_boundary(mlc_handle *h, double x1);
+// boundary, diagnostics and status_update of a step whose tendencies are zero
+int launch_boundary_step(mlc_handle *h, double x1);
 int launch_mkslice(mlc_handle *h, const mlc_slice_desc &s);
 int launch_fill(mlc_handle *h, const Buf &b, long long n, double value);
+// zeroes `count` (at most 6) arrays of n[m] elements
+int launch_zero(mlc_handle *h, const Buf *const *b, const long long *n, int count);
 int launch_fill64(mlc_handle *h, double *p, long long n, double value);
 int launch_waf_metrics(mlc_handle *h);
 int launch_terrain_check(mlc_handle *h, long long *nbad);

@@ -2323,7 +2323,11 @@ __device__ __forceinline__ double qx_check(int n) {
 // and east columns (corners excluded), one thread per (i, k); sn = 1: the
 // south and north rows (corners included), one thread per (j, k).  The two
 // run as separate launches in that order, as the reference's sequence needs
-// (a corner's outflow copy reads the value the west/east pass wrote).
+// (a corner's outflow copy reads the value the west/east pass wrote); bz is
+// the side.  A thread's work is one trip to memory: every load stands before
+// the first store, which could alias it (one field after the other, twice for
+// the two sides, was a chain of some twenty trips: 21.0 us per launch at
+// 151x127x35, where this takes 9.5).
 template <typename R>
 struct BdyVal {
   Dims d;
@@ -2358,91 +2362,88 @@ __device__ __forceinline__ void BdyVal<R>::run(const BdyVal &args_, int bx, int 
   double *__restrict__ pai = args_.pai;
   double *__restrict__ w = args_.w;
   R *__restrict__ ps = args_.ps;
+  const int sn = args_.sn, side = bz;
+  // the point of the wind normal to the boundary (pn) and of the one along it
+  // (pt), the boundary's cross point (cc) and its inner neighbour (cn)
+  long long pn, pt, cc, cn, c2;
+  bool cross, along;   // cross points (and the normal wind), the wind along it
+  if (!sn) {
+    const int i = m, jc = side == 0 ? 1 : jx - 1;
+    pn = d.at(side == 0 ? 1 : jx, i, k);
+    cc = d.at(jc, i, k);
+    pt = cc;
+    cn = d.at(side == 0 ? 2 : jx - 2, i, k);
+    c2 = d.at2(jc, i);
+    cross = i >= 2 && i <= iy - 2;
+    along = i >= 2 && i <= iy - 1;
+  } else {
+    const int j = m, ic = side == 0 ? 1 : iy - 1;
+    pn = d.at(j, side == 0 ? 1 : iy, k);
+    cc = d.at(j, ic, k);
+    pt = cc;                                       // u row: j in jde at i = ice
+    cn = d.at(j, side == 0 ? 2 : iy - 2, k);
+    c2 = d.at2(j, ic);
+    cross = j <= jx - 1;
+    along = true;
+  }
   auto lin = [&](const double *b0, const double *b1, long long c) {
     return x0 * b0[c] + x1 * b1[c];
   };
-  for (int side = 0; side < 2; ++side) {
-    if (!args_.sn) {
-      const int i = m;
-      const int jd = side == 0 ? 1 : jx;
-      const int jc = side == 0 ? 1 : jx - 1;
-      const int jn = side == 0 ? 2 : jx - 2;
-      const bool ici = i >= 2 && i <= iy - 2, idi = i >= 2 && i <= iy - 1;
-      const long long cd = d.at(jd, i, k), cc = d.at(jc, i, k), cn = d.at(jn, i, k);
-      if (ici && k == 1) ps[d.at2(jc, i)] = R(x0 * b.ps0[d.at2(jc, i)] + x1 * b.ps1[d.at2(jc, i)]);
-      if (ici) u[cd] = R(lin(b.u0, b.u1, cd));
-      if (idi) v[cc] = R(lin(b.v0, b.v1, cc));
-      if (ici) {
-        t[cc] = R(lin(b.t0, b.t1, cc));
-        pai[cc] = lin(b.pai0, b.pai1, cc);
-        args_.q.q[0][cc] = R(lin(b.qv0, b.qv1, cc));
-        if (pqc) args_.q.q[1][cc] = R(lin(b.qc0, b.qc1, cc));
-        if (pqi && args_.ipptls > 1) args_.q.q[2][cc] = R(lin(b.qi0, b.qi1, cc));
-        const double uu = u[cd];
-        const bool inflow = side == 0 ? uu > 0.0 : uu < 0.0;
-        // over the fixed maximum (10 species) with a guard: constant
-        // indices keep the argument struct out of scratch memory
+  R *wn = sn ? v : u, *wt = sn ? u : v;
+  const double *n0 = sn ? b.v0 : b.u0, *n1 = sn ? b.v1 : b.u1;
+  const double *t0 = sn ? b.u0 : b.v0, *t1 = sn ? b.u1 : b.v1;
+  R vn = R(0), vt = R(0), vb = R(0), nt = R(0), nqv = R(0), nqc = R(0), nqi = R(0), nps = R(0);
+  R qin[10], tin = R(0);
+  double npai = 0.0, win = 0.0;
+  const bool pqi2 = pqi && args_.ipptls > 1;
+  R *tke = args_.tke;
+  if (along) vt = R(lin(t0, t1, pt));
+  if (cross) {
+    vn = R(lin(n0, n1, pn));
+    nt = R(lin(b.t0, b.t1, cc));
+    npai = lin(b.pai0, b.pai1, cc);
+    nqv = R(lin(b.qv0, b.qv1, cc));
+    if (pqc) nqc = R(lin(b.qc0, b.qc1, cc));
+    if (pqi2) nqi = R(lin(b.qi0, b.qi1, cc));
+    // over the fixed maximum (10 species) with a guard: constant indices keep
+    // the argument struct out of scratch memory
 #pragma unroll
-        for (int n = 2; n <= 10; ++n) {
-          if (n > nqx || (pqc && n == 2) || (pqi && n == 3)) continue;
-          const R qxint = args_.q.q[n - 1][cn];
-          args_.q.q[n - 1][cc] = inflow ? R(qx_zero(n - 1)) : qxint;
-        }
-        w[cc] = inflow ? 0.0 : w[cn];
-        if (args_.tke) {
-          // TKE rows (Main/mod_bdycod.F90:1684-1694, :1742-1752): level 1 at
-          // tkemin; level k+1 (k = 2..kz) from the inflow sign of u(k) + u(k-1),
-          // u(k-1) being the value this stage writes at that level
-          R *tke = args_.tke;
-          if (k == 1) {
-            tke[cc] = R(args_.tkemin);
-          } else {
-            const double us = (double)u[cd] + (double)R(lin(b.u0, b.u1, cd - d.plane));
-            const bool tin = side == 0 ? us > 0.0 : us < 0.0;
-            tke[cc + d.plane] = tin ? R(args_.tkemin) : tke[cn + d.plane];
-          }
-        }
-      }
+    for (int n = 2; n <= 10; ++n)
+      if (n <= nqx) qin[n - 1] = args_.q.q[n - 1][cn];
+    win = w[cn];
+    if (tke && k > 1) {
+      vb = R(lin(n0, n1, pn - d.plane));
+      tin = tke[cn + d.plane];
+    }
+    if (k == 1) nps = R(lin(b.ps0, b.ps1, c2));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (along) wt[pt] = vt;
+  if (!cross) return;
+  wn[pn] = vn;
+  t[cc] = nt;
+  pai[cc] = npai;
+  args_.q.q[0][cc] = nqv;
+  if (pqc) args_.q.q[1][cc] = nqc;
+  if (pqi2) args_.q.q[2][cc] = nqi;
+  const bool inflow = side == 0 ? (double)vn > 0.0 : (double)vn < 0.0;
+#pragma unroll
+  for (int n = 2; n <= 10; ++n) {
+    if (n > nqx || (pqc && n == 2) || (pqi && n == 3)) continue;
+    args_.q.q[n - 1][cc] = inflow ? R(qx_zero(n - 1)) : qin[n - 1];
+  }
+  w[cc] = inflow ? 0.0 : win;
+  if (k == 1) ps[c2] = nps;
+  if (tke) {
+    // TKE rows (Main/mod_bdycod.F90:1684-1694, :1742-1752, :1800-1810,
+    // :1858-1868): level 1 at tkemin; level k+1 (k = 2..kz) from the inflow
+    // sign of the normal wind's sum over k and k-1
+    if (k == 1) {
+      tke[cc] = R(args_.tkemin);
     } else {
-      const int j = m;
-      const int id = side == 0 ? 1 : iy;
-      const int ic = side == 0 ? 1 : iy - 1;
-      const int in = side == 0 ? 2 : iy - 2;
-      const bool jce = j <= jx - 1;
-      const long long cdu = d.at(j, ic, k);          // u row: j in jde at i = ice
-      const long long cdv = d.at(j, id, k), cc = d.at(j, ic, k), cn = d.at(j, in, k);
-      if (jce && k == 1) ps[d.at2(j, ic)] = R(x0 * b.ps0[d.at2(j, ic)] + x1 * b.ps1[d.at2(j, ic)]);
-      u[cdu] = R(lin(b.u0, b.u1, cdu));
-      if (jce) {
-        v[cdv] = R(lin(b.v0, b.v1, cdv));
-        t[cc] = R(lin(b.t0, b.t1, cc));
-        pai[cc] = lin(b.pai0, b.pai1, cc);
-        args_.q.q[0][cc] = R(lin(b.qv0, b.qv1, cc));
-        if (pqc) args_.q.q[1][cc] = R(lin(b.qc0, b.qc1, cc));
-        if (pqi && args_.ipptls > 1) args_.q.q[2][cc] = R(lin(b.qi0, b.qi1, cc));
-        const double vv = v[cdv];
-        const bool inflow = side == 0 ? vv > 0.0 : vv < 0.0;
-        // over the fixed maximum (10 species) with a guard: constant
-        // indices keep the argument struct out of scratch memory
-#pragma unroll
-        for (int n = 2; n <= 10; ++n) {
-          if (n > nqx || (pqc && n == 2) || (pqi && n == 3)) continue;
-          const R qxint = args_.q.q[n - 1][cn];
-          args_.q.q[n - 1][cc] = inflow ? R(qx_zero(n - 1)) : qxint;
-        }
-        w[cc] = inflow ? 0.0 : w[cn];
-        if (args_.tke) {
-          // (Main/mod_bdycod.F90:1800-1810, :1858-1868), j over jce
-          R *tke = args_.tke;
-          if (k == 1) {
-            tke[cc] = R(args_.tkemin);
-          } else {
-            const double vs = (double)v[cdv] + (double)R(lin(b.v0, b.v1, cdv - d.plane));
-            const bool tin = side == 0 ? vs > 0.0 : vs < 0.0;
-            tke[cc + d.plane] = tin ? R(args_.tkemin) : tke[cn + d.plane];
-          }
-        }
-      }
+      const double ws = (double)vn + (double)vb;
+      const bool in2 = side == 0 ? ws > 0.0 : ws < 0.0;
+      tke[cc + d.plane] = in2 ? R(args_.tkemin) : tin;
     }
   }
 }
@@ -2483,42 +2484,76 @@ __device__ __forceinline__ void BdyRelax<R>::run(const BdyRelax &args_, int bx, 
   R *__restrict__ t = args_.t;
   double *__restrict__ pai = args_.pai;
   double *__restrict__ w = args_.w;
-  if (args_.top_nudge) {
+  // The weights decide which points change; those points' fields are then
+  // loaded together and stored together.  (One field after the other, each
+  // behind its own branch and the last one's store: 28.5 us at 151x127x35;
+  // this 21.2.)
+  const double xu = u_pt ? b.xfu[c] : -1.0, xv = v_pt ? b.xfv[c] : -1.0;
+  const double xc = c_pt ? b.xfc[c] : -1.0;
+  const bool top = args_.top_nudge && k <= args_.nztop;
+  const bool wtop = args_.top_nudge && k == 2 && c_pt;
+  const bool fu = u_pt && (top || xu >= 0.0), fv = v_pt && (top || xv >= 0.0);
+  const bool fc = c_pt && xc >= 0.0, ft = c_pt && (top || fc);
+  const bool pqc = args_.ipptls > 0 && args_.present_qc;
+  const bool pqi = args_.ipptls > 1 && args_.present_qi;
+  const double dta = args_.dta;
+  double xt = 0.0, uv = 0.0, ub = 0.0, vv = 0.0, vb = 0.0, tv = 0.0, tb = 0.0, wv = 0.0;
+  double pv = 0.0, pb = 0.0, q0 = 0.0, q0b = 0.0, q1 = 0.0, q1b = 0.0, q2 = 0.0, q2b = 0.0;
+  auto ext = [&](const double *b0, const double *b1) { return (x0 * b0[c] + x1 * b1[c]); };
+  if (top) xt = b.tnudge[k - 1];
+  if (fu) {
+    uv = (double)u[c];
+    ub = ext(b.u0, b.u1);
+  }
+  if (fv) {
+    vv = (double)v[c];
+    vb = ext(b.v0, b.v1);
+  }
+  if (ft) {
+    tv = (double)t[c];
+    tb = ext(b.t0, b.t1);
+  }
+  if (fc || wtop) wv = w[c];
+  if (fc) {
+    pv = pai[c];
+    pb = ext(b.pai0, b.pai1);
+    q0 = (double)args_.q.q[0][c];
+    q0b = ext(b.qv0, b.qv1);
+    if (pqc) {
+      q1 = (double)args_.q.q[1][c];
+      q1b = ext(b.qc0, b.qc1);
+    }
+    if (pqi) {
+      q2 = (double)args_.q.q[2][c];
+      q2b = ext(b.qi0, b.qi1);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  auto relax = [&](double f, double xf, double fext) { return (1.0 - xf) * f + xf * fext; };
+  if (top) {
     const double trtau = 1.0 / (2.0 * 3600.0);
+    const double xf = xt * trtau * dta;
+    tv = (double)R(relax(tv, xf, tb));
+    uv = (double)R(relax(uv, xf, ub));
+    vv = (double)R(relax(vv, xf, vb));
+  }
+  if (wtop) {
     const double wrtau = 1.0 / (3600.0 / 4.0);
-    const double dta = args_.dta;
-    if (c_pt && k == 2) {
-      const double fext = 0.0 * w[c];
-      const double xf = wrtau * dta;
-      w[c] = (1.0 - xf) * w[c] + xf * fext;
-    }
-    if (k <= args_.nztop) {
-      const double xf = b.tnudge[k - 1] * trtau * dta;
-      if (c_pt) t[c] = R((1.0 - xf) * (double)t[c] + xf * (x0 * b.t0[c] + x1 * b.t1[c]));
-      if (u_pt) u[c] = R((1.0 - xf) * (double)u[c] + xf * (x0 * b.u0[c] + x1 * b.u1[c]));
-      if (v_pt) v[c] = R((1.0 - xf) * (double)v[c] + xf * (x0 * b.v0[c] + x1 * b.v1[c]));
-    }
+    const double fext = 0.0 * wv;
+    const double xf = wrtau * dta;
+    wv = (1.0 - xf) * wv + xf * fext;
   }
-  auto relax = [&](double fv, double xf, const double *b0, const double *b1) {
-    const double fext = (x0 * b0[c] + x1 * b1[c]);
-    return (1.0 - xf) * fv + xf * fext;
-  };
-  if (u_pt && b.xfu[c] >= 0.0) u[c] = R(relax(u[c], b.xfu[c], b.u0, b.u1));
-  if (v_pt && b.xfv[c] >= 0.0) v[c] = R(relax(v[c], b.xfv[c], b.v0, b.v1));
-  if (c_pt) {
-    const double xf = b.xfc[c];
-    if (xf >= 0.0) {
-      t[c] = R(relax(t[c], xf, b.t0, b.t1));
-      pai[c] = relax(pai[c], xf, b.pai0, b.pai1);
-      args_.q.q[0][c] = R(relax(args_.q.q[0][c], xf, b.qv0, b.qv1));
-      w[c] = (1.0 - xf) * w[c] + xf * w[c] * 0.0;
-      if (args_.ipptls > 0) {
-        if (args_.present_qc) args_.q.q[1][c] = R(relax(args_.q.q[1][c], xf, b.qc0, b.qc1));
-        if (args_.ipptls > 1 && args_.present_qi)
-          args_.q.q[2][c] = R(relax(args_.q.q[2][c], xf, b.qi0, b.qi1));
-      }
-    }
+  if (fu) u[c] = xu >= 0.0 ? R(relax(uv, xu, ub)) : R(uv);
+  if (fv) v[c] = xv >= 0.0 ? R(relax(vv, xv, vb)) : R(vv);
+  if (ft) t[c] = fc ? R(relax(tv, xc, tb)) : R(tv);
+  if (fc) {
+    pai[c] = relax(pv, xc, pb);
+    args_.q.q[0][c] = R(relax(q0, xc, q0b));
+    if (pqc) args_.q.q[1][c] = R(relax(q1, xc, q1b));
+    if (pqi) args_.q.q[2][c] = R(relax(q2, xc, q2b));
+    wv = (1.0 - xc) * wv + xc * wv * 0.0;
   }
+  if (fc || wtop) w[c] = wv;
 }
 
 // Spectral nudging of one field (mospectral_nudge, Main/mod_bdycod.F90:
@@ -2667,25 +2702,46 @@ __device__ __forceinline__ void Slice<R>::run(const Slice &args_, int bx, int by
     const double ptr = s_ptrop[lane];
     for (int k = 1 + wv; k <= kz; k += kSliceWaves) {
       const long long c = d.at(j, i, k);
+      // one trip to memory per level: its loads stand before its stores,
+      // which could alias them (43.8 -> 29.7 us per call at 97x83x30, where a
+      // SIMD has less than one wave)
+      const double pa = a.pai[c], pb = a.pai[k >= 2 ? c - P : c + P];
+      const double pk = (double)a.p[c], tk = (double)a.t[c];
+      R qv[10] = {}, qs = R(1), ze = R(0);
+      double rho = 0.0, w0 = 0.0, w1 = 0.0;
+      if (inner || k == 1) rho = (double)a.rho[c];
+      if (inner) {
+#pragma unroll
+        for (int n = 0; n < 10; ++n)
+          if (n < a.nqx) qv[n] = a.q.q[n][c];
+        qs = a.qsat[c];
+        w0 = a.w[c];
+        w1 = a.w[c + P];
+        if (a.ibltyp == 1) ze = a.zeta[c];
+      }
+      __builtin_amdgcn_sched_barrier(0);
       if (k >= 2) {
-        a.pf[c] = kP00 * pow(0.5 * (a.pai[c] + a.pai[c - P]), kCpovr);
+        a.pf[c] = kP00 * pow(0.5 * (pa + pb), kCpovr);
       } else {
-        const double pf2 = kP00 * pow(0.5 * (a.pai[c + P] + a.pai[c]), kCpovr);
-        a.pf[c] = pf2 - kEgrav * (double)a.rho[c] * (a.zetaf[c] - a.zetaf[c + P]);
+        const double pf2 = kP00 * pow(0.5 * (pb + pa), kCpovr);
+        a.pf[c] = pf2 - kEgrav * rho * (a.zetaf[c] - a.zetaf[c + P]);
         a.pf[c + (long long)kz * P] = (double)a.ps[c2];
       }
-      const double pk = (double)a.p[c];
-      a.th[c] = (double)a.t[c] * pow(kP00 / pk, rovcp);
+      a.th[c] = tk * pow(kP00 / pk, rovcp);
       if (!inner) continue;
 #pragma unroll
-      for (int n = 0; n < 10; ++n)
-        if (n < a.nqx && a.q.q[n][c] < R(qx_check(n))) a.q.q[n][c] = R(qx_zero(n));
-      const double r = (double)a.q.q[0][c] / (double)a.qsat[c];
+      for (int n = 0; n < 10; ++n) {
+        if (n < a.nqx && qv[n] < R(qx_check(n))) {
+          qv[n] = R(qx_zero(n));
+          a.q.q[n][c] = qv[n];
+        }
+      }
+      const double r = (double)qv[0] / (double)qs;
       a.rh[c] = fmin(fmax(r, a.rhmin), a.rhmax);
-      a.omega[c] = -kEgrav * (double)a.rho[c] * 0.5 * (a.w[c + P] + a.w[c]);
+      a.omega[c] = -kEgrav * rho * 0.5 * (w1 + w0);
       if (k >= 2 && k <= kz - 1) {
         if (pk < ptr && k > kt) kt = k;
-        if (a.ibltyp == 1 && (double)a.zeta[c] > 5000.0 && k > kp) kp = k;
+        if (a.ibltyp == 1 && (double)ze > 5000.0 && k > kp) kp = k;
         if (a.icldmstrat == 1 && pk > 70000.0 && k < k7) k7 = k;
       }
     }
@@ -2761,7 +2817,8 @@ __device__ __forceinline__ double pfwsat(double t, double p) {
 }
 
 // flags: 1 = dycore tail (:1121-1125), 2 = diagnostics p, rho, qsat
-// (:348-352), 4 = status update (:1410-1438).  Pointwise on cross points.
+// (:348-352), 4 = status update (:1410-1438), 64 = its tendencies are zero and
+// not read.  Pointwise on cross points.
 // p comes from the double Exner function in both forms.
 // flags = 16: the three in one pass for a physics-off step, whose
 // tendencies are zero: status_update's additions x + dtinc*0 leave t and q
@@ -2889,8 +2946,10 @@ __device__ __forceinline__ void Tail<R>::run(const Tail &args_, int bx, int by, 
   if (flags & 2) {
     pp = R(pow(pa, kCpovr) * kP00);
     p[c] = pp;
-    rho[c] = pp / (R(kRgas) * tt);
-    qsat[c] = R(pfwsat((double)tt, (double)pp));
+    if (!(flags & 4)) {
+      rho[c] = pp / (R(kRgas) * tt);
+      qsat[c] = R(pfwsat((double)tt, (double)pp));
+    }
   }
   if (flags & 32) {
     // restart (Main/mod_init.F90:951-955): tvirt from water vapour alone,
@@ -2908,14 +2967,15 @@ __device__ __forceinline__ void Tail<R>::run(const Tail &args_, int bx, int by, 
   if (flags & 4) {
     if (!(flags & 2)) pp = p[c];
     if (interior) {
-      tt = tt + dtinc * tten[c];
+      const bool still = flags & 64;       // every tendency is zero
+      tt = tt + dtinc * (still ? R(0) : tten[c]);
       t[c] = tt;
-      ux[c] = ux[c] + dtinc * uten[c];
-      vx[c] = vx[c] + dtinc * vten[c];
+      ux[c] = ux[c] + dtinc * (still ? R(0) : uten[c]);
+      vx[c] = vx[c] + dtinc * (still ? R(0) : vten[c]);
 #pragma unroll
       for (int n = 0; n < 10; ++n) {
         if (n < nqx) {
-          R a = q.q[n][c] + dtinc * q.qt[n][c];
+          R a = q.q[n][c] + dtinc * (still ? R(0) : q.qt[n][c]);
           if (a < R(qcheck[n])) a = R(qzero[n]);
           q.q[n][c] = a;
         }
@@ -2932,7 +2992,9 @@ __device__ __forceinline__ void Tail<R>::run(const Tail &args_, int bx, int by, 
 // extrapolate_surface_pressure (:1592-1606) on interior columns.  With
 // from_exner, Tv(kz-1), Tv(kz) and p(kz) are formed from theta_v and the
 // Exner function as the dycore tail and the diagnostics form them (the
-// physics-off step runs this before its one-pass tail).
+// physics-off step runs this before its one-pass tail); with from_exner = 2
+// from T (in tvirt), the species and the Exner function, as temp_to_tvirt
+// and the diagnostics form them.
 template <typename R>
 struct SurfacePressure {
   Dims d;
@@ -2943,6 +3005,8 @@ struct SurfacePressure {
   const double * tetav;
   const double * pai;
   int from_exner;
+  QPtrs<R> q;          // from_exner = 2
+  int ipptls;
   static __device__ __forceinline__ void run(const SurfacePressure &args_, int bx, int by, int bz);
 };
 
@@ -2960,7 +3024,11 @@ __device__ __forceinline__ void SurfacePressure<R>::run(const SurfacePressure &a
   const int kz = d.kz;
   const long long ck = d.at(j, i, kz), cm = ck - d.plane;
   R tvm, tvk, pk;
-  if (args_.from_exner) {
+  if (args_.from_exner == 2) {
+    tvm = tvirt[cm] * tv_factor(args_.q, cm, args_.ipptls);
+    tvk = tvirt[ck] * tv_factor(args_.q, ck, args_.ipptls);
+    pk = R(pow(args_.pai[ck], kCpovr) * kP00);
+  } else if (args_.from_exner) {
     const double pak = args_.pai[ck];
     tvm = R(args_.tetav[cm] * args_.pai[cm]);
     tvk = R(args_.tetav[ck] * pak);
@@ -3075,6 +3143,22 @@ __device__ __forceinline__ void Fill<R>::run(const Fill &args_, int bx, int by, 
   const long long stride = args_.nblk * blockDim.x;
   for (long long m = idx; m < n; m += stride) p[m] = R(value);
 }
+
+// Zeroes several arrays in one launch, by = the array; their sizes are multiples
+// of 16 bytes (rows of 32 elements).  A launch per array took 3 to 4 us each
+// whatever its size (97x83x30, twelve arrays in five launches: 21 -> 9.8 us).
+constexpr int kMaxZero = 6;
+struct FillZero {
+  double2 *p[kMaxZero];
+  long long n[kMaxZero];   // 16-byte words
+  long long nblk;
+  static __device__ __forceinline__ void run(const FillZero &a, int bx, int by, int bz) {
+    double2 *__restrict__ p = a.p[by];
+    const long long n = a.n[by], stride = a.nblk * blockDim.x;
+    for (long long m = (long long)bx * blockDim.x + threadIdx.x; m < n; m += stride)
+      p[m] = make_double2(0.0, 0.0);
+  }
+};
 
 // ---------------------------------------------------------------------------
 // Error-free transformations for the compensated budget sums.
@@ -3266,6 +3350,7 @@ template <typename S, int GF, int GD> struct XcdOrder<WafVerticalMixed<S, GF, GD
 };
 template <typename R> struct XcdOrder<Tail<R>> { static constexpr bool value = false; };
 template <typename R> struct XcdOrder<Fill<R>> { static constexpr bool value = false; };
+template <> struct XcdOrder<FillZero> { static constexpr bool value = false; };
 template <typename R> struct XcdOrder<SurfacePressure<R>> { static constexpr bool value = false; };
 template <typename R> struct XcdOrder<BdyVal<R>> { static constexpr bool value = false; };
 template <typename R> struct XcdOrder<SpecNudge<R>> { static constexpr bool value = false; };
@@ -3798,7 +3883,7 @@ static int tail(mlc_handle *h, double dtinc, int flags) {
              h->rho.as<R>(), h->qsat.as<R>(), h->cur_adv(A_UX).as<R>(),
              h->cur_adv(A_VX).as<R>(), h->tten.as<R>(), h->uten.as<R>(),
              h->vten.as<R>(), dtinc, flags);
-  if ((flags & 2) && !(flags & 32))   // a restart keeps the saved ps
+  if ((flags & 2) && !(flags & (32 | 64)))   // a restart keeps the saved ps
     MLC_EMIT(K_PS, SurfacePressure<R>, grid_from2(d, d.jc2, d.ic2, 1), kBlock, 0,
                d, h->tvirt.as<R>(), h->zeta.as<R>(), h->p.as<R>(),
                h->ps.as<R>(), nullptr, nullptr, 0);
@@ -3813,7 +3898,15 @@ static int tail(mlc_handle *h, double dtinc, int flags) {
 }
 
 template <typename R>
-static int lbc(mlc_handle *h, double x1) {
+static int tracer_update(mlc_handle *h, double dtinc);
+
+// boundary(); `step` = 0.  In a whole physics-off step (step = 1) the
+// diagnostics and status_update follow with zero tendencies: temp_to_tvirt's
+// Tv and theta_v, of which only the surface pressure sees anything before
+// status_update forms them again, are formed there, and the three pointwise
+// passes become one (151x127x35: 3 x 15.9 us -> 19.5).
+template <typename R>
+static int lbc(mlc_handle *h, double x1, int step) {
   const Dims d = h->d;
   const LbcData bd = {h->lbc.ps0, h->lbc.ps1, h->lbc.u0, h->lbc.u1, h->lbc.v0, h->lbc.v1,
                       h->lbc.t0, h->lbc.t1, h->lbc.pai0, h->lbc.pai1, h->lbc.qv0,
@@ -3825,8 +3918,8 @@ static int lbc(mlc_handle *h, double x1) {
   const dim3 b256(256, 1, 1);
   for (int sn = 0; sn < 2; ++sn) {
     const int n_along = sn ? d.jx : d.iy;
-    const dim3 g((unsigned)((n_along + 256) / 256), (unsigned)d.kz, 1);
-    MLC_EMIT(K_LBC, BdyVal<R>, g, b256, 0, d, bd, u, v, t, pai, h->w, qptrs<R>(h),
+    const dim3 g((unsigned)((n_along + 64) / 64), (unsigned)d.kz, 2);
+    MLC_EMIT(K_LBC, BdyVal<R>, g, dim3(64, 1, 1), 0, d, bd, u, v, t, pai, h->w, qptrs<R>(h),
              h->ps.as<R>(), x1, h->g.nqx, h->g.ipptls, L.present_qc, L.present_qi, sn,
              h->s_tkex >= 0 ? h->tke.as<R>() : nullptr, h->tkemin);
   }
@@ -3865,11 +3958,19 @@ static int lbc(mlc_handle *h, double x1) {
   MLC_EMIT(K_LBC, StaggerIn<R>, grid_cross(d, snch), kBlock, 0, d, u, v, (const double *)h->w,
            h->fmzf.as<R>(), h->s.as<R>(), h->cur_adv(A_UX).as<R>(), h->cur_adv(A_VX).as<R>(),
            h->cur_adv(A_WX).as<R>(), 1, zmet(h, 4), skc);
-  return tail<R>(h, 0.0, 8);
+  if (!step) return tail<R>(h, 0.0, 8);
+  MLC_EMIT(K_PS, SurfacePressure<R>, grid_from2(d, d.jc2, d.ic2, 1), kBlock, 0, d, t,
+           h->zeta.as<R>(), nullptr, h->ps.as<R>(), nullptr, pai, 2, qptrs<R>(h),
+           h->g.ipptls);
+  int rc = tail<R>(h, h->g.dtsec, 2 | 4 | 64);
+  return rc ? rc : tracer_update<R>(h, h->g.dtsec);
 }
 
 int launch_boundary(mlc_handle *h, double x1) {
-  return h->mixed ? lbc<float>(h, x1) : lbc<double>(h, x1);
+  return h->mixed ? lbc<float>(h, x1, 0) : lbc<double>(h, x1, 0);
+}
+int launch_boundary_step(mlc_handle *h, double x1) {
+  return h->mixed ? lbc<float>(h, x1, 1) : lbc<double>(h, x1, 1);
 }
 
 template <typename R>
@@ -3959,6 +4060,17 @@ static int fill_t(mlc_handle *h, R *p, long long n, double value) {
 int launch_fill(mlc_handle *h, const Buf &b, long long n, double value) {
   return b.es == 4 ? fill_t<float>(h, b.as<float>(), n, value)
                    : fill_t<double>(h, b.as<double>(), n, value);
+}
+int launch_zero(mlc_handle *h, const Buf *const *b, const long long *n, int count) {
+  FillZero a{};
+  long long most = 0;
+  for (int m = 0; m < count; ++m) {
+    a.p[m] = b[m]->as<double2>();
+    a.n[m] = n[m] * b[m]->es / 16;
+    most = std::max(most, a.n[m]);
+  }
+  a.nblk = std::min((most + 255) / 256, 16384LL);
+  return emit(h, K_FILL, dim3((unsigned)a.nblk, (unsigned)count), dim3(256), 0, a);
 }
 int launch_fill64(mlc_handle *h, double *p, long long n, double value) {
   return fill_t<double>(h, p, n, value);
