@@ -1,6 +1,7 @@
 // C-ABI of libmoloch_hip: handle lifecycle, host<->device transfers of
 // Fortran-bounded boxes, init_moloch's derived metrics and the step
 // orchestration of moloch() (Main/mod_moloch.F90:312-446).
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -550,19 +551,23 @@ static int build_bdy_tables(mlc_handle *h) {
 }
 
 // Fields per thread of the vertical WAF for nf fields on cross columns that
-// make `waves` wavefronts.  A SIMD runs its waves' levels one after the
-// other, and a level costs about 0.7 of a field on top of the fields (s and
-// the metric ratios), so the cost is the waves of the fullest of the chip's
-// 1024 SIMDs times (fields per wave + 0.7): few fields per wave where the
-// domain leaves SIMDs idle or unevenly filled, four where it fills them.
-// Measured, us per call at 4 / 2 / 1: 64x64x23 20.2 / 16.2 / 13.8,
-// 151x127x35 57 / 47 / 53, 500x100x60 144 / 128 / 162, 256x256x41 109 / 128 / 145.
+// make `waves` wavefronts.  A level costs about 0.95 of a field on top of the
+// fields (s and the metric ratios).  The first wave of a SIMD costs 1.7 of a
+// further one, whose waits it shares; the waves are those of the fullest of
+// the chip's 1024 SIMDs and of the average one, halfway, since full and idle
+// SIMDs share the memory.  Few fields per wave where the domain leaves SIMDs
+// idle or unevenly filled, four where it fills them.  Measured, us per call at
+// 4 / 2 / 1 fields: 64x64x23 20 / 16 / 13.6, 100x50x30 mixed 28.8 / 18.3 / 16.0,
+// 97x83x30 with 14 fields 32.7 / 30.3 / 26.6, 151x127x35 61 / 44 / 50,
+// 500x100x60 162 / 133 / 160, 256x256x41 121 / 123 / 145.
 static int wafv_rule(long long waves, int nf) {
   int best = 4;
   double cost = 0.0;
   for (int g = 4; g >= 1; g /= 2) {
     const int groups = (nf + g - 1) / g;
-    const double c = (double)((waves * groups + 1023) / 1024) * ((double)nf / groups + 0.7);
+    const double load = (double)(waves * groups) / 1024.0;
+    const double fill = std::max(1.0, 0.5 * (load + std::ceil(load)));
+    const double c = ((double)nf / groups + 0.95) * (fill + 0.7);
     if (g == 4 || c < cost) {
       best = g;
       cost = c;
@@ -651,6 +656,13 @@ void launch_shapes(mlc_handle *const *h, int n) {
   rows_rule(h, n, &rows, &group);
   for (int m = 0; m < n; ++m) {
     h[m]->tune.wafv_group = wafv;
+    // Past one round of the chip (four waves per SIMD) the groups of a tile
+    // run next to each other on one XCD and read s and the metric ratios from
+    // its L2: 512x512x41 mixed 284 -> 260 us per call, 8 x 128x128x30 188 -> 180.
+    // Within a round they run beside each other anyway, and the plain order
+    // spreads the longer waves better: 256x256x41 mixed 64 against 75,
+    // 151x127x35 44 against 51.
+    h[m]->tune.wafv_near = waves * ((nf + wafv - 1) / wafv) > 4096;
     h[m]->tune.waf_rows = rows;
     h[m]->tune.waf_group = group;
     // a domain that fills the chip with one level chunk keeps 8 levels in the

@@ -82,6 +82,21 @@ __device__ __forceinline__ double waf_b(double r) {
 __device__ __forceinline__ float waf_b(float r) {
   return fmaxf(0.0f, fminf(2.0f, fmaxf(r, fminf(2.0f * r, 1.0f))));
 }
+// The same as instructions: fmin and fmax first quiet an r that comes from a
+// select.  One instruction in 47 of a vertical face; the horizontal faces'
+// scheduling loses more than that by the fixed block.
+__device__ __forceinline__ double waf_b_v(double r) {
+  double m;
+  asm("v_max_f64 %0, %1, %2\n\tv_min_f64 %0, %0, 2.0\n\tv_max_f64 %0, %0, 0"
+      : "=&v"(m) : "v"(r), "v"(fmin(2.0 * r, 1.0)));
+  return m;
+}
+__device__ __forceinline__ float waf_b_v(float r) {
+  float m;
+  asm("v_max_f32 %0, %1, %2\n\tv_min_f32 %0, 2.0, %0\n\tv_max_f32 %0, 0, %0"
+      : "=&v"(m) : "v"(r), "v"(fminf(2.0f * r, 1.0f)));
+  return m;
+}
 
 // num / den as the limiter needs it, for |den| >= FlowLim::den(): correctly
 // rounded between -4 and 4, past them some value of the same sign beyond 2
@@ -1139,7 +1154,9 @@ __device__ __forceinline__ void StaggerIn<R>::run(const StaggerIn &args_, int bx
 // level: 47 vector instructions per face instead of 74.  Measured per call,
 // one domain alone: 64x64x23 38.0 -> 13.8 us, 151x127x35 68.1 -> 47.5,
 // 500x100x60 156 -> 128, 256x256x41 FP64 114 -> 109 (4.5 TB/s over its 23
-// arrays) and mixed 83.9 -> 66.3.
+// arrays) and mixed 83.9 -> 66.3.  Two levels per iteration, under rocprofv3:
+// 24x20x10 7.3 -> 6.3 us, 64x64x23 15.4 -> 13.8, 151x127x35 47.2 -> 43.2,
+// 256x256x41 mixed 68.3 -> 60.6.
 template <typename T>
 struct WafFace {       // the field-independent part of a face flux
   T az, half;          // |s dtrdz|, 0.5 s
@@ -1153,7 +1170,7 @@ struct WafFace {       // the field-independent part of a face flux
   // face kk+1 from xm, x0, x1, x2 = x(kk-1), x(kk), x(kk+1), x(kk+2), with
   // the k1/k1p1 clamps of :870-880 in the caller's operands
   __device__ __forceinline__ T flux(T xm, T x0, T x1, T x2) const {
-    const T b = waf_b(flow_param_sel(up ? x1 - x2 : xm - x0, x0 - x1));
+    const T b = waf_b_v(flow_param_sel(up ? x1 - x2 : xm - x0, x0 - x1));
     const T zphi = waf_phi(az, b, up);
     return half * ((T(1) + zphi) * x1 + (T(1) - zphi) * x0);
   }
@@ -1168,8 +1185,13 @@ struct WafVertical {
   const S * zrfmd;
   double dtrdz_;
   int nf;                      // fields in the batch
-  int ngroups;                 // bz = 0 .. ngroups-1: near-equal groups of at most G fields
-  static __device__ __forceinline__ void run(const WafVertical &args_, int bx, int by, int bz);
+  int ngroups;                 // near-equal groups of at most G fields
+  int near;                    // 1: bx counts the groups of a tile first; 0: bz is the group
+  // group = 0 .. ngroups-1 of tile (bx, by)
+  static __device__ __forceinline__ void group(const WafVertical &args_, int bx, int by, int grp);
+  static __device__ __forceinline__ void run(const WafVertical &a, int bx, int by, int bz) {
+    group(a, a.near ? bx / a.ngroups : bx, by, a.near ? bx % a.ngroups : bz);
+  }
 };
 
 // The column of the N fields f0 .. f0+N-1; the per-level loads of s, zrfmu
@@ -1218,6 +1240,8 @@ __device__ __forceinline__ void waf_column(const Dims &d, const AdvPtrs<T> &ap, 
   // (a load issued after a store would wait for the store as well).
   auto level = [&](int k, auto emit_, auto last_) __attribute__((always_inline)) {
     constexpr bool emit = decltype(emit_)::value, last = decltype(last_)::value;
+    // unrolled, a level's requests stay in it
+    if constexpr (N < 3 || sizeof(T) == 4) __builtin_amdgcn_sched_barrier(0);
     T x3[N];
     S ns = S(0), nu = S(0), nd = S(0);
     if constexpr (!last) {
@@ -1275,7 +1299,20 @@ __device__ __forceinline__ void waf_column(const Dims &d, const AdvPtrs<T> &ap, 
   // the second half step's first face has x(0) = x(1)
 #pragma unroll
   for (int g = 0; g < N; ++g) ym[g] = y0[g];
-  for (int k = 3; k < kz; ++k) level(k, std::true_type{}, std::false_type{});
+  // Two levels per iteration halve the moves of the windows (107 instructions
+  // per field and level instead of 123); with three or more double fields the
+  // registers would take the third wave per SIMD (a spill of 10 cost 112 ->
+  // 120 us at 256x256x41).
+  int k = 3;
+  if constexpr (N < 3 || sizeof(T) == 4) {
+    for (; k + 1 < kz; k += 2) {
+      level(k, std::true_type{}, std::false_type{});
+      level(k + 1, std::true_type{}, std::false_type{});
+    }
+    if (k < kz) level(k, std::true_type{}, std::false_type{});
+  } else {
+    for (; k < kz; ++k) level(k, std::true_type{}, std::false_type{});
+  }
   level(kz, std::true_type{}, std::true_type{});
   // wz2(kz-1) and wz2(kz): y0, y1 = wz1(kz-1), wz1(kz); s_k = s(kz+1)
   const WafFace<T> fb(s_1, dtrdz);
@@ -1289,8 +1326,8 @@ __device__ __forceinline__ void waf_column(const Dims &d, const AdvPtrs<T> &ap, 
 }
 
 template <typename T, typename S, int G>
-__device__ __forceinline__ void WafVertical<T, S, G>::run(const WafVertical &args_, int bx, int by,
-                                                          int bz) {
+__device__ __forceinline__ void WafVertical<T, S, G>::group(const WafVertical &args_, int bx,
+                                                            int by, int bz) {
   const Dims d = args_.d;
   const int j = 1 + bx * TJ + threadIdx.x;
   const int i = 1 + by * TI + threadIdx.y;
@@ -1815,12 +1852,14 @@ template <typename S, int GF, int GD>
 struct WafVerticalMixed {
   WafVertical<float, S, GF> f;
   WafVertical<double, S, GD> p;
-  int ngf;                     // blocks with bz < ngf run the float batch
   static __device__ __forceinline__ void run(const WafVerticalMixed &a, int bx, int by, int bz) {
-    if (bz < a.ngf)
-      WafVertical<float, S, GF>::run(a.f, bx, by, bz);
+    // the float batch's groups, then the double batch's
+    const int ng = a.f.ngroups + a.p.ngroups;
+    const int grp = a.f.near ? bx % ng : bz, tx = a.f.near ? bx / ng : bx;
+    if (grp < a.f.ngroups)
+      WafVertical<float, S, GF>::group(a.f, tx, by, grp);
     else
-      WafVertical<double, S, GD>::run(a.p, bx, by, bz - a.ngf);
+      WafVertical<double, S, GD>::group(a.p, tx, by, grp - a.f.ngroups);
   }
 };
 
@@ -3342,12 +3381,6 @@ void chunks(const Dims &d, int target, int *nch, int *kc) {
     prof_push(h, slot, ea_, eb_);                                                 \
   } while (0)
 
-template <typename T, typename S, int G> struct XcdOrder<WafVertical<T, S, G>> {
-  static constexpr bool value = false;
-};
-template <typename S, int GF, int GD> struct XcdOrder<WafVerticalMixed<S, GF, GD>> {
-  static constexpr bool value = false;
-};
 template <typename R> struct XcdOrder<Tail<R>> { static constexpr bool value = false; };
 template <typename R> struct XcdOrder<Fill<R>> { static constexpr bool value = false; };
 template <> struct XcdOrder<FillZero> { static constexpr bool value = false; };
@@ -3370,7 +3403,8 @@ template <> struct MinWaves<Tail<float>> { static constexpr int value = 6; };
 // Launch (or, while the handle records, append to its launch record) one
 // stage on the handle's stream.
 template <class A>
-int emit(mlc_handle *h, int slot, dim3 grid, dim3 block, size_t lds, const A &a) {
+int emit(mlc_handle *h, int slot, dim3 grid, dim3 block, size_t lds, const A &a,
+         bool xcd = XcdOrder<A>::value) {
   if (grid.x == 0 || grid.y == 0 || grid.z == 0) return MLC_OK;
   if (h->rec) {
     LaunchRec r;
@@ -3386,7 +3420,7 @@ int emit(mlc_handle *h, int slot, dim3 grid, dim3 block, size_t lds, const A &a)
   }
   hipEvent_t ea, eb;
   prof_events(h, slot, &ea, &eb);
-  void (*kern)(A) = h->tune.xcd_map && XcdOrder<A>::value &&
+  void (*kern)(A) = h->tune.xcd_map && xcd &&
                             (unsigned long long)grid.x * grid.y * grid.z >= 16
                         ? k_one_xcd<A>
                         : k_one<A>;
@@ -3541,6 +3575,12 @@ static int waf_vertical(mlc_handle *h, const Dims &d, const AdvPtrs<R> &vb, int 
                         const AdvPtrs<double> &vp, int np, double dtrdz) {
   using WafVRR = WafVertical<R, R, G>;
   using WafVDR = WafVertical<double, R, G>;
+  const int near = h->tune.wafv_near;
+  auto grid = [&](int ng) {
+    dim3 g = grid_cross(d, near ? 1 : ng);
+    if (near) g.x *= (unsigned)ng;
+    return g;
+  };
   if constexpr (sizeof(R) == 4) {
     if (np && (h->tune.mixed_merge & 1)) {
       // float and double batches in one launch
@@ -3548,19 +3588,18 @@ static int waf_vertical(mlc_handle *h, const Dims &d, const AdvPtrs<R> &vb, int 
       using WafVM = WafVerticalMixed<R, G, GD>;
       const int ngf = (nb + G - 1) / G, ngd = (np + GD - 1) / GD;
       const WafVM a{WafVertical<float, R, G>{d, vb, h->s.as<R>(), h->zrfmu.as<R>(),
-                                             h->zrfmd.as<R>(), dtrdz, nb, ngf},
+                                             h->zrfmd.as<R>(), dtrdz, nb, ngf, near},
                     WafVertical<double, R, GD>{d, vp, h->s.as<R>(), h->zrfmu.as<R>(),
-                                               h->zrfmd.as<R>(), dtrdz, np, ngd},
-                    ngf};
-      return emit(h, K_WAF_V, grid_cross(d, ngf + ngd), kBlock, 0, a);
+                                               h->zrfmd.as<R>(), dtrdz, np, ngd, near}};
+      return emit(h, K_WAF_V, grid(ngf + ngd), kBlock, 0, a, near);
     }
   }
-  MLC_EMIT(K_WAF_V, WafVRR, grid_cross(d, (nb + G - 1) / G), kBlock, 0, d, vb,
-           h->s.as<R>(), h->zrfmu.as<R>(), h->zrfmd.as<R>(), dtrdz, nb, (nb + G - 1) / G);
-  if (np)
-    MLC_EMIT(K_WAF_V, WafVDR, grid_cross(d, (np + G - 1) / G), kBlock, 0, d, vp,
-             h->s.as<R>(), h->zrfmu.as<R>(), h->zrfmd.as<R>(), dtrdz, np, (np + G - 1) / G);
-  return MLC_OK;
+  const int ngb = (nb + G - 1) / G, ngp = (np + G - 1) / G;
+  const WafVRR b{d, vb, h->s.as<R>(), h->zrfmu.as<R>(), h->zrfmd.as<R>(), dtrdz, nb, ngb, near};
+  int rc = emit(h, K_WAF_V, grid(ngb), kBlock, 0, b, near);
+  if (rc || !np) return rc;
+  const WafVDR p{d, vp, h->s.as<R>(), h->zrfmu.as<R>(), h->zrfmd.as<R>(), dtrdz, np, ngp, near};
+  return emit(h, K_WAF_V, grid(ngp), kBlock, 0, p, near);
 }
 
 template <typename R, int TR, int PER>

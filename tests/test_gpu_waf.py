@@ -6,8 +6,8 @@ import pytest
 
 import oracle_api as O
 from regcm_amd import synth
-from regcm_amd.moloch import (MLC_VAR_WAF_GROUP, MLC_VAR_WAF_H, MLC_VAR_WAF_ROWS,
-                              MLC_VAR_WAFV_GROUP, Moloch)
+from regcm_amd.moloch import (MLC_MIXED, MLC_VAR_WAF_GROUP, MLC_VAR_WAF_H, MLC_VAR_WAF_ROWS,
+                              MLC_VAR_WAFV_GROUP, Moloch, relative_l2)
 
 pytestmark = pytest.mark.gpu
 
@@ -86,3 +86,27 @@ def test_extreme_values():
         for n in range(2):
             assert np.array_equal(a[n], b[n], equal_nan=True), \
                 f"tracer {n}: {np.count_nonzero(~((a[n] == b[n]) | (np.isnan(a[n]) & np.isnan(b[n]))))}"
+
+
+@pytest.mark.parametrize("group", [1, 2, 4])
+def test_groups_of_a_tile_next_to_each_other(group):
+    """More waves than one round of the chip: the vertical pass counts a tile's
+    field groups first (25 fields, so that the domain stays small)."""
+    g, f, _ = synth.config("small", jx=201, iy=190, kz=5, ntr=15, nadv=1, nsound=1)
+    check(g, f, {MLC_VAR_WAFV_GROUP: group}, f"groups first, {group} per thread")
+
+
+def test_groups_of_a_tile_next_to_each_other_mixed():
+    """The same with the float and the double batch in one launch, against the
+    oracle within the mixed form's error (one float rounding per operation)."""
+    print("[waf] groups first, mixed", flush=True)
+    g, f, _ = synth.config("small", jx=201, iy=190, kz=5, ntr=15, nadv=1, nsound=1)
+    ref = O.copy_fields(f)
+    O.moloch_steps(g, ref, 1)
+    with Moloch(g, MLC_MIXED) as m:
+        m.load(f)
+        m.init_moloch()
+        m.moloch(1)
+        m.synchronize()
+        for n, tol in (("u", 1e-5), ("tetav", 1e-6), ("pai", 1e-7), ("qx", 1e-5), ("trac", 1e-5)):
+            assert relative_l2(owned(g, n, ref[n]), owned(g, n, m.get(n))) < tol, n
