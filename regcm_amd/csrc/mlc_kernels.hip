@@ -117,7 +117,13 @@ __device__ __forceinline__ double waf_ratio(double num, double den) {
   const double r = __builtin_fma(-den, q, num);
   return __builtin_amdgcn_div_fixup(__builtin_fma(r, y, q), den, num);
 }
-__device__ __forceinline__ float waf_ratio(float num, float den) {
+// The hardware's float reciprocal flushes a result below 2^-126 to zero, so a
+// float denominator of 2^126 and more needs both operands a quarter as large.
+// (A num below 2^-124 loses bits by that; its quotient is below 1e-22.)  Two
+// instructions per face: the mixed vertical pass 60.0 -> 61.0 us at 256x256x41,
+// the horizontal one unchanged.
+__device__ __forceinline__ float waf_ratio(float num_, float den_) {
+  const float num = 0.25f * num_, den = 0.25f * den_;
   float y = __builtin_amdgcn_rcpf(den);
   y = __builtin_fmaf(__builtin_fmaf(-den, y, 1.0f), y, y);
   float q = fmaxf(fminf(num * y, 4.0f), -4.0f);
@@ -1151,7 +1157,7 @@ __device__ __forceinline__ void StaggerIn<R>::run(const StaggerIn &args_, int bx
 // last-level cache and the 2F + 3 arrays do.  So a face is branch-free, its
 // limiter is min/max instructions, its division leaves out the scaling
 // (waf_ratio) and the parts that do not depend on the field are formed once per
-// level: 47 vector instructions per face instead of 74.  Measured per call,
+// level: 47 vector instructions per face (49 in float) instead of 74.  Measured per call,
 // one domain alone: 64x64x23 38.0 -> 13.8 us, 151x127x35 68.1 -> 47.5,
 // 500x100x60 156 -> 128, 256x256x41 FP64 114 -> 109 (4.5 TB/s over its 23
 // arrays) and mixed 83.9 -> 66.3.  Two levels per iteration, under rocprofv3:
