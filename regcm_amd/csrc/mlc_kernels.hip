@@ -3697,9 +3697,9 @@ static int waf_rows(mlc_handle *h, const Dims &d, AdvPtrs<R> hb, AdvPtrs<R> wzb,
   const R *tanrot = h->tanrot.as<R>();
   if (nb) {
     const int ng = (nb + G - 1) / G;
-    // ux and vx go first, into one group of at least two fields, which then
-    // applies the curvature terms
-    const bool fuse = cux >= 0 && cvx == cux + 1 && nb / ng >= 2;
+    // ux and vx go first, into the first group, which then applies the curvature
+    // terms; it holds ceil(nb / ng) fields, at least two whenever nb has both
+    const bool fuse = cux >= 0 && cvx == cux + 1 && (nb + ng - 1) / ng >= 2;
     if (fuse)
       for (int m = 0; m < 2; ++m) {
         std::swap(hb.src[m], hb.src[cux + m]);
