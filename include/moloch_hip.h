@@ -210,30 +210,33 @@ int mlc_kernel_stats(mlc_handle *h, int slot, long long *launches,
                      double *total_ms);
 
 /* Launch-shape variants of a stage.  Every variant of a stage gives
- * bit-identical results; their speed depends on the domain shape.  No
- * reference counterpart (a GPU launch choice). */
+ * bit-identical results; their speed depends on the domain shape.  A knob
+ * of a form that does not run is kept and has no effect until that form is
+ * chosen.  No reference counterpart (a GPU launch choice). */
 #define MLC_VAR_WAF_H 0       /* horizontal WAF: 0 row-streaming (default), 1 LDS tile */
 #define MLC_VAR_WAF_ROWS 1    /* row-streaming WAF: i rows per wavefront, 4..256 (by domain size) */
 #define MLC_VAR_WAF_GROUP 2   /* row-streaming WAF: fields per lane, 2 or 4 (by domain size) */
 #define MLC_VAR_LEVEL_CHUNK 3 /* divergence (and momentum, unless MLC_VAR_MOM_CHUNK is set):
                                  levels per thread, 1..kz (by domain size) */
 #define MLC_VAR_COLUMN 4      /* column solve: 0 LDS three-phase, 1 streamed, 2 LDS with
-                                 level chunks in registers (default; kz > 64 runs 0) */
+                                 level chunks in registers (default; kz > 128 runs 1) */
 #define MLC_VAR_WAFV_GROUP 5  /* vertical WAF: fields per thread, 1, 2 or 4 (by domain
                                  size) */
 #define MLC_VAR_XCD_MAP 6     /* single-domain launches: 1 XCD-contiguous tile order (default), 0 plain */
 #define MLC_VAR_WAF_TILE 7    /* LDS-tile WAF: output rows per tile, 4 or 8 (default 8 in FP64, 4 mixed) */
 #define MLC_VAR_WAF_HGROUP 8  /* LDS-tile WAF: fields per block, 0 = the whole batch (default) */
-#define MLC_VAR_COLUMN_J 9    /* chunked column solve: columns per block, 16, 32 or 64 (up
-                                 to 42 levels; by domain size) */
+#define MLC_VAR_COLUMN_J 9    /* chunked column solve: columns per block, 16, 32 (up to
+                                 64 levels) or 64 (up to 42); by domain size */
 #define MLC_VAR_MIXED_MERGE 10 /* mixed form: float and double WAF batches in one launch,
-                                 bit 0 vertical (default 1), bit 1 horizontal as two block
-                                 ranges, bit 2 horizontal in the same blocks (one coefficient
-                                 setup; whole batch per block) */
+                                 bit 0 vertical (default 1); of the horizontal LDS-tile form
+                                 (MLC_VAR_WAF_H 1) bit 1 as two block ranges, bit 2 in the
+                                 same blocks (one coefficient setup; whole batch per block).
+                                 The row-streaming form always takes two launches */
 #define MLC_VAR_TERRAIN 11    /* terrain metrics formed from the orography instead of streamed
                                  from the uploaded 3-D arrays, as a mask of stages: 1
                                  divergence, 2 column solve, 4 advection staggering, 8
-                                 horizontal WAF.  mlc_init sets 7 (FP64) or 6 (mixed) when the
+                                 horizontal WAF in its LDS-tile form (MLC_VAR_WAF_H 1; the
+                                 row-streaming form streams them).  mlc_init sets 7 (FP64) or 6 (mixed) when the
                                  formed values equal every uploaded one (MLC_PARAM_MO_H), else
                                  0; a non-zero mask otherwise is MLC_E_STATE.  Same bits
                                  either way. */
@@ -246,8 +249,8 @@ int mlc_set_variant(mlc_handle *h, int stage, int value);
 int mlc_get_variant(const mlc_handle *h, int stage);
 
 /* Autotuner: times whole steps of this domain under the launch-shape
- * variants (coordinate descent over the stages above, each candidate timed
- * over nsteps steps after one warm-up step) and keeps a candidate only when
+ * variants (coordinate descent over the stages above, each candidate that
+ * changes what runs timed over nsteps steps after one warm-up step) and keeps a candidate only when
  * it is at least 1% faster than the value it would replace.  The
  * state is snapshotted on the device first and restored afterwards, so the
  * call leaves the domain exactly as it found it.  *ms_per_step (may be

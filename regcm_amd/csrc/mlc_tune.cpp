@@ -7,6 +7,7 @@
 // stage's candidates with the other stages at their best so far: restore,
 // one warm-up step, nsteps timed steps between two events on the handle's
 // stream.  It ends by restoring the snapshot and keeping the best shapes.
+#include <algorithm>
 #include <cstring>
 #include <vector>
 
@@ -107,10 +108,22 @@ int autotune(mlc_handle *h, int nsteps, double *best_ms) {
   };
 
   constexpr double kTuneMargin = 0.01;
+  // What a knob's value comes to under the other knobs: values that come to the
+  // same run the same launches, and only one of them is timed.  A knob of the
+  // horizontal WAF form that does not run comes to 0 whatever its value.
   struct Knob {
     int *slot;
     std::vector<int> values;
+    int (*effect)(const mlc_handle *, int);
   };
+  const auto plain = [](const mlc_handle *, int v) { return v; };
+  const auto rows_only = [](const mlc_handle *h, int v) { return h->tune.waf_h == 0 ? v : 0; };
+  const auto tile_only = [](const mlc_handle *h, int v) { return h->tune.waf_h == 1 ? v : 0; };
+  const auto chunked = [](const mlc_handle *h, int v) { return h->tune.column == 2 ? v : 0; };
+  const auto merged = [](const mlc_handle *h, int v) {
+    return h->mixed ? (h->tune.waf_h == 1 ? v : v & 1) : 0;
+  };
+  const auto formed = [](const mlc_handle *h, int v) { return h->tune.waf_h == 1 ? v : v & 7; };
   std::vector<int> chunk_vals;
   for (int c : {2, 4, 6, 8, 12, 16})
     if (c <= h->g.kz) chunk_vals.push_back(c);
@@ -123,25 +136,25 @@ int autotune(mlc_handle *h, int nsteps, double *best_ms) {
   for (int c : {1, 2, 4, 8})
     if (c <= h->g.kz) stag_vals.push_back(c);
   std::vector<Knob> knobs = {
-      {&h->tune.waf_h, {0, 1}},
-      {&h->tune.waf_rows, {4, 8, 12, 16, 32}},
-      {&h->tune.waf_group, {2, 4}},
-      {&h->tune.level_chunk, chunk_vals},
-      {&h->tune.mom_chunk, mom_vals},
-      {&h->tune.stag_chunk, stag_vals},
-      {&h->tune.column, {0, 1, 2}},
-      {&h->tune.wafv_group, {1, 2, 4}},
-      {&h->tune.xcd_map, {0, 1}},
-      {&h->tune.waf_tile, {4, 8}},
-      {&h->tune.waf_hgroup, {0, 1, 2, 4}},
-      {&h->tune.column_j, {16, 32, 64}},
-      {&h->tune.mixed_merge, {0, 1, 2, 3, 4, 5}},
+      {&h->tune.waf_h, {0, 1}, plain},
+      {&h->tune.waf_rows, {4, 8, 12, 16, 32}, rows_only},
+      {&h->tune.waf_group, {2, 4}, rows_only},
+      {&h->tune.level_chunk, chunk_vals, plain},
+      {&h->tune.mom_chunk, mom_vals, plain},
+      {&h->tune.stag_chunk, stag_vals, plain},
+      {&h->tune.column, {0, 1, 2}, plain},
+      {&h->tune.wafv_group, {1, 2, 4}, plain},
+      {&h->tune.xcd_map, {0, 1}, plain},
+      {&h->tune.waf_tile, {4, 8}, tile_only},
+      {&h->tune.waf_hgroup, {0, 1, 2, 4}, tile_only},
+      {&h->tune.column_j, {16, 32, 64}, chunked},
+      {&h->tune.mixed_merge, {0, 1, 2, 3, 4, 5}, merged},
   };
   // formed or streamed terrain metrics per stage (the same bits), where
   // mlc_init verified the formed ones: first, so the launch shapes are tuned
   // with it, and again last, for the shapes chosen
   if (h->zmet_ok) {
-    const Knob t{&h->tune.terrain, {0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15}};
+    const Knob t{&h->tune.terrain, {0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15}, formed};
     knobs.insert(knobs.begin(), t);
     knobs.push_back(t);
   }
@@ -154,9 +167,16 @@ int autotune(mlc_handle *h, int nsteps, double *best_ms) {
   for (auto &k : knobs) {
     const int keep = *k.slot;
     int arg = keep;
-    if ((rc = time_steps(&best))) return cleanup(rc);
+    std::vector<int> todo, seen = {k.effect(h, keep)};
     for (int v : k.values) {
-      if (v == keep) continue;
+      const int e = k.effect(h, v);
+      if (std::find(seen.begin(), seen.end(), e) != seen.end()) continue;
+      seen.push_back(e);
+      todo.push_back(v);
+    }
+    if (todo.empty()) continue;
+    if ((rc = time_steps(&best))) return cleanup(rc);
+    for (int v : todo) {
       *k.slot = v;
       double ms = 0.0;
       if ((rc = time_steps(&ms))) {
