@@ -656,13 +656,7 @@ void launch_shapes(mlc_handle *const *h, int n) {
   rows_rule(h, n, &rows, &group);
   for (int m = 0; m < n; ++m) {
     h[m]->tune.wafv_group = wafv;
-    // Past one round of the chip (four waves per SIMD) the groups of a tile
-    // run next to each other on one XCD and read s and the metric ratios from
-    // its L2: 512x512x41 mixed 284 -> 260 us per call, 8 x 128x128x30 188 -> 180.
-    // Within a round they run beside each other anyway, and the plain order
-    // spreads the longer waves better: 256x256x41 mixed 64 against 75,
-    // 151x127x35 44 against 51.
-    h[m]->tune.wafv_near = waves * ((nf + wafv - 1) / wafv) > 4096;
+    h[m]->tune.wafv_waves = waves;
     h[m]->tune.waf_rows = rows;
     h[m]->tune.waf_group = group;
     // a domain that fills the chip with one level chunk keeps 8 levels in the

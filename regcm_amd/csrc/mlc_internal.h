@@ -317,7 +317,7 @@ struct mlc_handle {
     int stag_chunk = 1;          // staggering passes: levels per thread
     int column = 2;              // column solve: 0 LDS three-phase, 1 streamed, 2 chunked
     int wafv_group = 4;          // vertical WAF: fields per thread (1, 2 or 4; launch_shapes)
-    int wafv_near = 0;           // vertical WAF: a tile's groups next to each other (launch_shapes)
+    long long wafv_waves = 0;    // vertical WAF: waves of one field group (launch_shapes)
     int xcd_map = 1;             // XCD-contiguous tile order of single-domain launches
     int waf_tile = 4;            // LDS-tile WAF: output rows per tile (4 or 8; FP64 starts at 8)
     int waf_hgroup = 0;          // LDS-tile WAF: fields per block (0 = the whole batch)

@@ -3581,10 +3581,19 @@ static int waf_vertical(mlc_handle *h, const Dims &d, const AdvPtrs<R> &vb, int 
                         const AdvPtrs<double> &vp, int np, double dtrdz) {
   using WafVRR = WafVertical<R, R, G>;
   using WafVDR = WafVertical<double, R, G>;
-  const int near = h->tune.wafv_near;
+  // Past one round of the chip (four waves per SIMD, five of one float field) the
+  // groups of a tile run next to each other on one XCD and read s and the metric
+  // ratios from its L2: us per call, plain order -> this, 512x512x41 mixed 284 ->
+  // 260, 8 x 128x128x30 188 -> 180, 200x200x30 one field per wave 88 -> 75,
+  // 256x256x41 two fields 122 -> 111.  Within a round they run beside each other
+  // anyway, and the plain order spreads the longer waves better: 256x256x41 mixed
+  // 64 against 75, 151x127x35 44 against 51, mixed with one field 33 against 38.
+  // By the groups that this call launches, however their size was chosen.
+  constexpr int kRound = G == 1 && sizeof(R) == 4 ? 5120 : 4096;
+  auto near = [&](int ng) { return h->tune.wafv_waves * ng > kRound ? 1 : 0; };
   auto grid = [&](int ng) {
-    dim3 g = grid_cross(d, near ? 1 : ng);
-    if (near) g.x *= (unsigned)ng;
+    dim3 g = grid_cross(d, near(ng) ? 1 : ng);
+    if (near(ng)) g.x *= (unsigned)ng;
     return g;
   };
   if constexpr (sizeof(R) == 4) {
@@ -3592,20 +3601,22 @@ static int waf_vertical(mlc_handle *h, const Dims &d, const AdvPtrs<R> &vb, int 
       // float and double batches in one launch
       constexpr int GD = G < 2 ? G : 2;
       using WafVM = WafVerticalMixed<R, G, GD>;
-      const int ngf = (nb + G - 1) / G, ngd = (np + GD - 1) / GD;
+      const int ngf = (nb + G - 1) / G, ngd = (np + GD - 1) / GD, nr = near(ngf + ngd);
       const WafVM a{WafVertical<float, R, G>{d, vb, h->s.as<R>(), h->zrfmu.as<R>(),
-                                             h->zrfmd.as<R>(), dtrdz, nb, ngf, near},
+                                             h->zrfmd.as<R>(), dtrdz, nb, ngf, nr},
                     WafVertical<double, R, GD>{d, vp, h->s.as<R>(), h->zrfmu.as<R>(),
-                                               h->zrfmd.as<R>(), dtrdz, np, ngd, near}};
-      return emit(h, K_WAF_V, grid(ngf + ngd), kBlock, 0, a, near);
+                                               h->zrfmd.as<R>(), dtrdz, np, ngd, nr}};
+      return emit(h, K_WAF_V, grid(ngf + ngd), kBlock, 0, a, nr);
     }
   }
   const int ngb = (nb + G - 1) / G, ngp = (np + G - 1) / G;
-  const WafVRR b{d, vb, h->s.as<R>(), h->zrfmu.as<R>(), h->zrfmd.as<R>(), dtrdz, nb, ngb, near};
-  int rc = emit(h, K_WAF_V, grid(ngb), kBlock, 0, b, near);
+  const WafVRR b{d, vb, h->s.as<R>(), h->zrfmu.as<R>(), h->zrfmd.as<R>(), dtrdz, nb, ngb,
+                 near(ngb)};
+  int rc = emit(h, K_WAF_V, grid(ngb), kBlock, 0, b, near(ngb));
   if (rc || !np) return rc;
-  const WafVDR p{d, vp, h->s.as<R>(), h->zrfmu.as<R>(), h->zrfmd.as<R>(), dtrdz, np, ngp, near};
-  return emit(h, K_WAF_V, grid(ngp), kBlock, 0, p, near);
+  const WafVDR p{d, vp, h->s.as<R>(), h->zrfmu.as<R>(), h->zrfmd.as<R>(), dtrdz, np, ngp,
+                 near(ngp)};
+  return emit(h, K_WAF_V, grid(ngp), kBlock, 0, p, near(ngp));
 }
 
 template <typename R, int TR, int PER>
