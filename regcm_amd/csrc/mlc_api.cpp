@@ -627,7 +627,13 @@ static void rows_rule(mlc_handle *const *h, int n, int *rows, int *group) {
 // It fits the measured times to 10% between one and seven blocks per CU
 // (momentum, us: 151x127x35 at 1 / 5 / 6 / 9 / 18 chunks 21.6 / 10.6 / 12.6 /
 // 12.1 / 11.4; 500x100x60 at 1 / 4 / 5 / 8 / 10 chunks 37.0 / 34.3 / 29.3 / 33.7
-// / 30.9; 64x64x23 at 1 / 12 / 23 chunks 15.7 / 4.8 / 4.8).
+// / 30.9; 64x64x23 at 1 / 12 / 23 chunks 15.7 / 4.8 / 4.8).  Domains that fill
+// the chip with whole columns take it too, momentum / divergence in us at 1 / 2
+// / 3 / 4 / 6 chunks (* the rule's): 256x256x41 FP64 30.7/32.4 27.7/24.4
+// *28.7/26.1 29.7/26.6 29.5/26.5, mixed 26.5/28.7 18.6/17.2 *20.1/15.0 20.5/15.1
+// 21.3/15.8; 288x288x41 FP64 51.9/42.0 *43.8/35.6 47.1/37.3 46.2/36.3 45.3/35.2;
+// 384x384x41 104/73 95/65 *91/59 91/60 91/62; 512x512x41 *161/128 160/129 159/129
+// 159/130 158/135, mixed *102/57 103/64 103/64 107/68 101/64.
 static int chunk_rule(long long blocks, int kz) {
   int best = kz;
   double cost = 0.0;
@@ -659,13 +665,9 @@ void launch_shapes(mlc_handle *const *h, int n) {
     h[m]->tune.wafv_waves = waves;
     h[m]->tune.waf_rows = rows;
     h[m]->tune.waf_group = group;
-    // a domain that fills the chip with one level chunk keeps 8 levels in the
-    // divergence, and in FP64 whole columns in the momentum update (31.7 us
-    // against 36.9 in four chunks at 256x256x41, where both stream from HBM)
-    const int kz = h[m]->g.kz, kc = chunk_rule(waves / 4, kz);
-    const bool full = waves >= 1024;
-    h[m]->tune.level_chunk = full ? (kz < 8 ? kz : 8) : kc;
-    h[m]->tune.mom_chunk = full && !h[m]->mixed ? kz : kc;
+    const int kc = chunk_rule(waves / 4, h[m]->g.kz);
+    h[m]->tune.level_chunk = kc;
+    h[m]->tune.mom_chunk = kc;
     // 16 columns per block while 32 leave CUs without one: 64x64x23 11.4 ->
     // 9.0 us, 100x50x30 mixed 11.8 -> 10.7; 151x127x35 loses, 20.7 -> 22.3
     h[m]->tune.column_j = columns <= 256 ? 16 : 32;
