@@ -104,24 +104,30 @@ def nadv_fields(g) -> int:
 
 
 def kernel_struct(slot: str, variants: dict, form: str, kz: int = 41,
-                  crm: int = 0) -> str | None:
+                  crm: int = 0, lrotllr: int = 0) -> str | None:
     """The argument-struct name rocprofv3 shows for a kernel slot's launch
     in the given launch shapes (as regcm_amd.profsum.short_name prints it);
-    crm = 1 on a doubly periodic domain (the horizontal WAF's own
-    instantiation)."""
+    the horizontal WAF has instantiations of its own for a doubly periodic
+    domain (crm = 1) and the rotated projection (lrotllr = 1)."""
     r = "double" if form == "fp64" else "float"
     per = 1 if crm else 0
     if slot == "sound_column":
-        if variants["column"] == 2:
-            cj = variants.get("column_j", 32)
+        tall = variants["column"] == 0 and kz > 63     # past the three-phase form's LDS
+        if variants["column"] == 2 or tall:
+            # the widest block that holds the column, at most the one asked for
+            cj = 16 if tall else variants.get("column_j", 32)
+            cj = 32 if cj == 64 and kz > 42 else cj
+            cj = 16 if cj == 32 and kz > 64 else cj
+            if kz > 128:
+                return f"SoundColumnStream<{r}>"
             ck = 256 // cj
-            cc = 6 if cj == 32 else 3          # levels per thread when kz <= 48
+            cc = {64: 11, 32: 6, 16: 3}[cj]    # levels per thread; 8 past kz = 48
             return f"SoundColumnChunk<{r},{cj},{ck},{cc if kz <= ck * cc else 8}>"
         base = {0: "SoundColumn", 1: "SoundColumnStream"}[variants["column"]]
         return f"{base}<{r}>"
     if slot == "waf_horizontal":
         if variants["waf_h"] == 0:
-            return f"WafRows<{r},{r},{variants['waf_group']}>"
+            return f"WafRows<{r},{r},{per},{1 if lrotllr and not crm else 0}>"
         if (form == "mixed" and variants.get("mixed_merge", 0) & 4
                 and variants.get("waf_hgroup", 0) == 0):
             return f"WafHorizontalFused<{r},{variants.get('waf_tile', 4)},{per}>"
@@ -130,7 +136,8 @@ def kernel_struct(slot: str, variants: dict, form: str, kz: int = 41,
         return f"WafHorizontal<{r},{r},{variants.get('waf_tile', 4)},{per}>"
     if slot == "waf_vertical":
         if form == "mixed" and variants.get("mixed_merge", 0) & 1:
-            return f"WafVerticalMixed<{r},{variants.get('wafv_group', 4)},2>"
+            gf = variants.get("wafv_group", 4)
+            return f"WafVerticalMixed<{r},{gf},{min(gf, 2)}>"
         return f"WafVertical<{r},{r},{variants.get('wafv_group', 4)}>"
     names = {"sound_div": "SoundDiv", "sound_momentum": "SoundMomentum",
              "adv_stagger_in": "StaggerIn", "adv_curvature": "Curvature",
@@ -139,12 +146,12 @@ def kernel_struct(slot: str, variants: dict, form: str, kz: int = 41,
 
 
 def read_traffic(slot: str, workload: str, variants: dict, form: str, kz: int = 41,
-                 crm: int = 0):
+                 crm: int = 0, lrotllr: int = 0):
     """HBM bytes per launch of the kernel of `slot` from the committed
     rocprofv3 counter summary (FETCH_SIZE + WRITE_SIZE, copy-kernel
     calibrated) for this workload and form, if there is one."""
     path = ROOT / "profiles" / f"pmc_traffic_{workload}_{form}.md"
-    name = kernel_struct(slot, variants, form, kz, crm)
+    name = kernel_struct(slot, variants, form, kz, crm, lrotllr)
     if not path.exists() or name is None:
         return None
     for line in path.read_text().splitlines():
@@ -682,7 +689,7 @@ def main() -> int:
         bpl = bpl / per_call
     achieved = (bpl / avg_s / 1e9) if bpl else None
     traffic = read_traffic(dname, args.workload, r["variants"], args.form, g.kz,
-                           getattr(g, "crm", 0))
+                           getattr(g, "crm", 0), g.lrotllr)
     out = {
         "metric": METRIC,
         "value": r["value"],
