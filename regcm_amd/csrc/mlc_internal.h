@@ -143,7 +143,9 @@ struct BdyWt {
 // within an ulp, and its exact remainder (Markstein's correction).  The
 // compiler's own division also scales both operands against overflow and
 // underflow: 11 dependent instructions against 6.  Zero, infinite and NaN
-// operands need v_div_fixup (recip).
+// operands need v_div_fixup (recip).  Against the division: the same bits for
+// 8.4e9 random operands and for the 32 mantissas next to all ones and to all
+// zeros at every exponent.
 __device__ __forceinline__ double recip_normal(double x) {
   double y = __builtin_amdgcn_rcp(x);
   double e = __builtin_fma(-x, y, 1.0);
@@ -162,8 +164,8 @@ __device__ __forceinline__ double recip(double x) {
 //   rfmzu(j,i,k) = 1/md_fmz(zitah(k), htu(j,i)),  rfmzv on htv
 // (md_fmz / md_fmz_h, Share/mod_zita.F90:135-141, 165-170), with the same
 // operations in the same order as the reference, so each value is the one
-// the caller computed.  The divisions are recip_normal, in the check too.  gzitap and bzitap are per-level tables; ht, htu, htv
-// are 2-D.  `on` is set only after mlc_init has compared the formula with
+// the caller computed.  The divisions are recip_normal, in the check too.
+// gzitap and bzitap are per-level tables; ht, htu, htv are 2-D.  `on` is set only after mlc_init has compared the formula with
 // every uploaded metric bit for bit, and then per stage; otherwise the
 // kernels stream the uploaded 3-D arrays.
 struct ZMet {

@@ -107,7 +107,8 @@ __device__ __forceinline__ float waf_b_v(float r) {
 // underflow; here the quotient is held within +-4 before the remainder is
 // formed, and a remainder can lose bits only for |num| below 1e-280 (1e-31 in
 // float), whose quotient is too small to change zphi = 1 + zamu b - b in its
-// last bit.
+// last bit.  Against the division: the same bits for 8.4e9 random pairs of
+// either type with quotients within +-4.
 __device__ __forceinline__ double waf_ratio(double num, double den) {
   double y = __builtin_amdgcn_rcp(den);
   double e = __builtin_fma(-den, y, 1.0);
@@ -485,15 +486,19 @@ __device__ __forceinline__ void SoundColumn<R>::run(const SoundColumn &args_, in
 // most CC levels of its column, whose z2, pai, metrics and tetavf stay in
 // registers, so LDS holds only the three tridiagonal arrays (zu, zd, rhs) and
 // level tables.  CJ columns per block (along j), CK threads per column;
-// requires kz <= CK * CC, and runs with the smallest CC that holds the column
-// (6 or 3 for kz <= 48, else 8) so that no thread carries unused levels.  Same
-// operations as SoundColumn.
+// requires kz <= CK * CC, and runs with the smallest CC built that holds the
+// column (6 or 3 for kz <= 48, else 8).  A thread owns kc = ceil(kz / CK) levels
+// and runs CC: the surplus ones load and compute at clamped or at the next
+// chunk's levels and store nothing (kz 41 and 60 have none; kz 30 owns 4 of 6 in
+// 32-column blocks and 2 of 3 in 16-column ones).  Same operations as
+// SoundColumn.
 //
-// Large domains are bound by memory: every array is read once, also across
-// the chunks (a thread passes its last level's values on through LDS), no
-// store stands before a load, and a few levels' loads are always in flight
-// within the registers of four waves per SIMD.  Small domains are bound by the
-// chain of kz divisions, which reads LDS a level ahead and takes the short
+// Large domains are bound by memory: a chunk's own levels are read once, none
+// again for its neighbour (a thread passes its last level's values on through
+// LDS), no store stands before a load, and a few levels' loads are always in flight
+// within the registers of four waves per SIMD (three of eight levels, two of
+// eleven).  Small domains run their phases one after the other, load, chain of
+// kz divisions and store; the chain reads LDS a level ahead and takes the short
 // reciprocal.  Measured per call, before (a chunk's neighbour level formed
 // twice, one level's inputs in flight, tetavf stored as it is formed) and
 // after: 256x256x41 FP64 49.2 -> 45.2 us (4.3 TB/s over its 9 arrays), mixed
@@ -3394,15 +3399,16 @@ template <typename R> struct XcdOrder<SurfacePressure<R>> { static constexpr boo
 template <typename R> struct XcdOrder<BdyVal<R>> { static constexpr bool value = false; };
 template <typename R> struct XcdOrder<SpecNudge<R>> { static constexpr bool value = false; };
 template <typename R> struct XcdOrder<Slice<R>> { static constexpr bool value = false; };
-// Slice<double> takes 152 VGPRs (3 waves per SIMD) unbounded; capped at 128
-// it spills 22 to scratch and still runs a 256 x 256 x 41 domain in one
-// round instead of 1.33 (170 -> 126 us).  Tail<float> reaches 6 without
-// spilling.
 // The column solve's loads and its chunk of every array, held for the update,
-// fit four waves per SIMD up to eight levels per thread.
+// fit four waves per SIMD up to six levels per thread (126 VGPRs), three at
+// eight (158) and two at eleven (210).
 template <typename R, int CJ, int CK, int CC> struct MinWaves<SoundColumnChunk<R, CJ, CK, CC>> {
   static constexpr int value = CC <= 6 ? 4 : CC <= 8 ? 3 : 2;
 };
+// Slice<double> takes 137 VGPRs (3 waves per SIMD) unbounded; capped at 128 it
+// spills 8 and runs a 256 x 256 x 41 domain in one round instead of 1.33: 90.9 ->
+// 82.2 us.  Domains of less or of several rounds pay the spills: 97x83x30 25.4 ->
+// 26.7, 512x512x41 351 -> 362.  Tail<float> reaches 6 without spilling.
 template <> struct MinWaves<Slice<double>> { static constexpr int value = 4; };
 template <> struct MinWaves<Tail<float>> { static constexpr int value = 6; };
 
