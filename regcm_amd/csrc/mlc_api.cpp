@@ -622,26 +622,28 @@ static void rows_rule(mlc_handle *const *h, int n, int *rows, int *group) {
 
 // Levels per thread of the level-chunked stages (divergence, momentum) on
 // `blocks` 64 x 4 tiles: the chunk of kz / n levels that minimises
-// (levels + 1) (1 + 0.8 (blocks per CU - 1)), a block's time being its levels
-// and one start, and a further block on the same CU adding 0.8 of its own.
-// It fits the measured times to 10% between one and seven blocks per CU
-// (momentum, us: 151x127x35 at 1 / 5 / 6 / 9 / 18 chunks 21.6 / 10.6 / 12.6 /
-// 12.1 / 11.4; 500x100x60 at 1 / 4 / 5 / 8 / 10 chunks 37.0 / 34.3 / 29.3 / 33.7
-// / 30.9; 64x64x23 at 1 / 12 / 23 chunks 15.7 / 4.8 / 4.8).  Domains that fill
-// the chip with whole columns take it too, momentum / divergence in us at 1 / 2
-// / 3 / 4 / 6 chunks (* the rule's): 256x256x41 FP64 30.7/32.4 27.7/24.4
-// *28.7/26.1 29.7/26.6 29.5/26.5, mixed 26.5/28.7 18.6/17.2 *20.1/15.0 20.5/15.1
-// 21.3/15.8; 288x288x41 FP64 51.9/42.0 *43.8/35.6 47.1/37.3 46.2/36.3 45.3/35.2;
-// 384x384x41 104/73 95/65 *91/59 91/60 91/62; 512x512x41 *161/128 160/129 159/129
-// 159/130 158/135, mixed *102/57 103/64 103/64 107/68 101/64.
-static int chunk_rule(long long blocks, int kz) {
+// (levels + 1) (1 + a (blocks per CU - 1)), a block's time being its levels and
+// one start, and a further block on the same CU adding a of its own: 0.8, but
+// all of it in the FP64 momentum update, which one block per CU keeps at the
+// memory's rate.  It fits the measured times to 10% between one and seven blocks
+// per CU (momentum, us: 151x127x35 at 1 / 5 / 6 / 9 / 18 chunks 21.6 / 10.6 /
+// 12.6 / 12.1 / 11.4; 500x100x60 at 1 / 4 / 5 / 8 / 10 chunks 37.0 / 34.3 / 29.3 /
+// 33.7 / 30.9; 64x64x23 at 1 / 12 / 23 chunks 15.7 / 4.8 / 4.8).  One round of
+// whole columns that nearly fills the chip is the FP64 momentum's best, and the
+// worst past that round.  Steps in us, levels of the divergence / the momentum:
+//   FP64    225x225x41   8/41 1621, 14/14 1651     256x256x41  14/41 1878, 14/14 1916
+//           256x256x30   8/30 1447, 10/10 1469     256x256x60   8/60 3019, 15/15 3094
+//           272x272x41   8/41 2458, 14/14 2247     384x384x41   8/41 4931, 14/14 4735
+//           200x200x60   8/60 2262,   8/8 2250     272x272x60   8/60 4069, 20/20 3654
+//   mixed   256x256x41   8/41 1362, 14/14 1307     320x320x41   8/41 2044, 14/14 2013
+static int chunk_rule(long long blocks, int kz, double a) {
   int best = kz;
   double cost = 0.0;
   for (int n = 1; n <= kz; ++n) {
     const int kc = (kz + n - 1) / n;
     if ((kz + kc - 1) / kc != n) continue;
-    const double c = (kc + 1.0) * (1.0 + 0.8 * (double)((blocks * n + 255) / 256 - 1));
-    if (cost == 0.0 || c < cost) {
+    const double c = (kc + 1.0) * (1.0 + a * (double)((blocks * n + 255) / 256 - 1));
+    if (cost == 0.0 || c <= cost) {       // the shorter of equals: 200x200x41 1603 -> 1578
       cost = c;
       best = kc;
     }
@@ -665,9 +667,8 @@ void launch_shapes(mlc_handle *const *h, int n) {
     h[m]->tune.wafv_waves = waves;
     h[m]->tune.waf_rows = rows;
     h[m]->tune.waf_group = group;
-    const int kc = chunk_rule(waves / 4, h[m]->g.kz);
-    h[m]->tune.level_chunk = kc;
-    h[m]->tune.mom_chunk = kc;
+    h[m]->tune.level_chunk = chunk_rule(waves / 4, h[m]->g.kz, 0.8);
+    h[m]->tune.mom_chunk = chunk_rule(waves / 4, h[m]->g.kz, h[m]->mixed ? 0.8 : 1.0);
     // 16 columns per block while 32 leave CUs without one: 64x64x23 11.4 ->
     // 9.0 us, 100x50x30 mixed 11.8 -> 10.7; 151x127x35 loses, 20.7 -> 22.3
     h[m]->tune.column_j = columns <= 256 ? 16 : 32;
