@@ -629,19 +629,24 @@ static void rows_rule(mlc_handle *const *h, int n, int *rows, int *group) {
 // per CU (momentum, us: 151x127x35 at 1 / 5 / 6 / 9 / 18 chunks 21.6 / 10.6 /
 // 12.6 / 12.1 / 11.4; 500x100x60 at 1 / 4 / 5 / 8 / 10 chunks 37.0 / 34.3 / 29.3 /
 // 33.7 / 30.9; 64x64x23 at 1 / 12 / 23 chunks 15.7 / 4.8 / 4.8).  One round of
-// whole columns that nearly fills the chip is the FP64 momentum's best, and the
-// worst past that round.  Steps in us, levels of the divergence / the momentum:
-//   FP64    225x225x41   8/41 1621, 14/14 1651     256x256x41  14/41 1878, 14/14 1916
-//           256x256x30   8/30 1447, 10/10 1469     256x256x60   8/60 3019, 15/15 3094
-//           272x272x41   8/41 2458, 14/14 2247     384x384x41   8/41 4931, 14/14 4735
-//           200x200x60   8/60 2262,   8/8 2250     272x272x60   8/60 4069, 20/20 3654
-//   mixed   256x256x41   8/41 1362, 14/14 1307     320x320x41   8/41 2044, 14/14 2013
+// whole columns (a block per CU) that nearly fills the chip is the FP64
+// momentum's best, and the worst past that round: there a chunk has at most 10
+// levels, and its rows are still cached when the tiles beside it run.  Steps in
+// us, levels of the divergence / the momentum:
+//   FP64    225x225x41   8/41 1621, 14/14 1651     200x200x60   8/60 2262,   8/8 2250
+//           256x256x41  14/41 1878,   7/7 1925     256x256x60   8/60 3019, 15/15 3094
+//           272x272x41   8/41 2458,   7/7 2266     272x272x60   8/60 4069, 10/10 3635
+//           384x384x41   8/41 4931, 14/14 4735, 7/7 4686
+//           512x512x41  41/41 9089, 14/14 8913, 7/7 8792
+//   mixed   256x256x41   8/41 1362, 14/14 1307     384x384x41 14/14 3160,   7/7 3119
+//   24 uneven domains of 23 to 41 levels, FP64 whole columns in both 32.8 ms, a
+//   third of the column 32.7, 8 levels 31.6; mixed 22.1, 21.8, 20.7
 static int chunk_rule(long long blocks, int kz, double a) {
   int best = kz;
   double cost = 0.0;
   for (int n = 1; n <= kz; ++n) {
     const int kc = (kz + n - 1) / n;
-    if ((kz + kc - 1) / kc != n) continue;
+    if ((kz + kc - 1) / kc != n || (blocks > 256 && kc > 10)) continue;
     const double c = (kc + 1.0) * (1.0 + a * (double)((blocks * n + 255) / 256 - 1));
     if (cost == 0.0 || c <= cost) {       // the shorter of equals: 200x200x41 1603 -> 1578
       cost = c;
