@@ -236,7 +236,8 @@ int mlc_kernel_stats(mlc_handle *h, int slot, long long *launches,
                                  from the uploaded 3-D arrays, as a mask of stages: 1
                                  divergence, 2 column solve, 4 advection staggering, 8
                                  horizontal WAF in its LDS-tile form (MLC_VAR_WAF_H 1; the
-                                 row-streaming form streams them).  mlc_init sets 7 (FP64) or 6 (mixed) when the
+                                 row-streaming form streams them).  mlc_init sets 7 (FP64)
+                                 or 6 (mixed) when the
                                  formed values equal every uploaded one (MLC_PARAM_MO_H), else
                                  0; a non-zero mask otherwise is MLC_E_STATE.  Same bits
                                  either way. */
@@ -250,7 +251,8 @@ int mlc_get_variant(const mlc_handle *h, int stage);
 
 /* Autotuner: times whole steps of this domain under the launch-shape
  * variants (coordinate descent over the stages above, each candidate that
- * changes what runs timed over nsteps steps after one warm-up step) and keeps a candidate only when
+ * changes what runs timed over nsteps steps after one warm-up step) and keeps
+ * a candidate only when
  * it is at least 1% faster than the value it would replace.  The
  * state is snapshotted on the device first and restored afterwards, so the
  * call leaves the domain exactly as it found it.  *ms_per_step (may be

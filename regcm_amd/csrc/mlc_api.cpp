@@ -559,7 +559,7 @@ static int build_bdy_tables(mlc_handle *h) {
 // idle or unevenly filled, four where it fills them.  Measured, us per call at
 // 4 / 2 / 1 fields: 64x64x23 20 / 16 / 13.6, 100x50x30 mixed 28.8 / 18.3 / 16.0,
 // 97x83x30 with 14 fields 32.7 / 30.3 / 26.6, 151x127x35 61 / 44 / 50,
-// 500x100x60 162 / 133 / 160, 256x256x41 121 / 123 / 145.
+// 500x100x60 162 / 133 / 160, 256x256x41 111 / 111 / 142.
 static int wafv_rule(long long waves, int nf) {
   int best = 4;
   double cost = 0.0;
