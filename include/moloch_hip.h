@@ -252,11 +252,10 @@ int mlc_get_variant(const mlc_handle *h, int stage);
 /* Autotuner: times whole steps of this domain under the launch-shape
  * variants (coordinate descent over the stages above, each candidate that
  * changes what runs timed over nsteps steps after one warm-up step) and keeps
- * a candidate only when
- * it is at least 1% faster than the value it would replace.  The
- * state is snapshotted on the device first and restored afterwards, so the
- * call leaves the domain exactly as it found it.  *ms_per_step (may be
- * null) receives the best step time.  Synchronous. */
+ * a candidate only when it is at least 1% faster than the value it would
+ * replace.  The state is snapshotted on the device first and restored
+ * afterwards, so the call leaves the domain exactly as it found it.
+ * *ms_per_step (may be null) receives the best step time.  Synchronous. */
 int mlc_autotune(mlc_handle *h, int nsteps, double *ms_per_step);
 
 /* Number of grid points of the step metric: the cross points times kz,

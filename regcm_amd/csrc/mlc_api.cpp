@@ -639,6 +639,9 @@ static void rows_rule(mlc_handle *const *h, int n, int *rows, int *group) {
 //           384x384x41   8/41 4931, 14/14 4735, 7/7 4686
 //           512x512x41  41/41 9089, 14/14 8913, 7/7 8792
 //   mixed   256x256x41   8/41 1362, 14/14 1307     384x384x41 14/14 3160,   7/7 3119
+//   either side of one block per CU, 256 columns by 252, 256, 260 and 272 rows:
+//           FP64  14/41 1873 1909 2218 2375, 6/6 or 7/7 1904 1943 2042 2107
+//           mixed 14/14 1292 1310 1394 1437, 6/6 or 7/7 1302 1322 1390 1431
 //   24 uneven domains of 23 to 41 levels, FP64 whole columns in both 32.8 ms, a
 //   third of the column 32.7, 8 levels 31.6; mixed 22.1, 21.8, 20.7
 static int chunk_rule(long long blocks, int kz, double a) {
